@@ -59,6 +59,8 @@ enum {
   UA_FLAG_GATES_F32 = 16,  /* bf16 ops: static_src, static_dest and the gradients dsrc, ddest are float32 tensors (the
                               reference allocates dstatic_src in static_src.dtype and accepts float32 gates next to
                               bf16 q, k, v: universal_attention_kernel.py:825-829).  float32 ops: always so. */
+  UA_FLAG_FORWARD_ONLY = 32, /* ua_fused_fwd(_strided): no backward will use this forward state; the working tensors only
+                              a backward reads are not written */
   UA_FLAG_PRUNE = 2        /* fused ops: skip (key, query) pairs whose softmax weight is provably below 2^-48 because
                               of the accumulated decay (no counterpart in the reference, which visits every pair).
                               The bound uses the largest key and query norms of the head; results change by less
@@ -91,6 +93,13 @@ typedef struct ua_chunked {
   void* ptr;
   int64_t stride_z, stride_t, stride_d, stride_i;
 } ua_chunked;
+
+/* The gates static_src / static_dest [b,h,L], or their gradients: element (b, h, t) of either at
+ * b*stride_b + h*stride_h + t*stride_t (elements of their dtype, see UA_FLAG_GATES_F32). */
+typedef struct ua_gates {
+  void *src, *dest;
+  int64_t stride_b, stride_h, stride_t;
+} ua_gates;
 
 int ua_version(void);
 /* Hash of the sources this library was compiled from (csrc/ and this header), as computed by the build script; a host
@@ -141,6 +150,11 @@ int ua_bwd(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_r
 int ua_fused_fwd(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_rows* xq, const void* static_src,
                  const void* static_dest, void* O, float* lse, void* ws, size_t ws_bytes, ua_stream_t stream);
 
+/* The same with every tensor described by its strides, for callers that hold views (a fused gate projection [b,L,2h],
+ * heads in another order): O rows as in xq (stride_outer and inner_len are not used: row t at t * stride_inner). */
+int ua_fused_fwd_strided(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_rows* xq, const ua_gates* gates,
+                         const ua_rows* O, float* lse, void* ws, size_t ws_bytes, ua_stream_t stream);
+
 /* The fused forward for callers that cannot allocate or supply device scratch (code under HIP graph capture, serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments and results as ua_fused_fwd
  * minus the workspace: the scratch is a device array inside the library, UA_NOALLOC_SCRATCH_BYTES per GPU, held from
@@ -161,6 +175,12 @@ int ua_fused_fwd_noalloc(const ua_desc* desc, const ua_rows* kc, const ua_rows* 
 int ua_fused_bwd(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_rows* xq, const void* static_src,
                  const void* static_dest, const void* O, const float* lse, const void* dO, void* dkc, void* dvc,
                  void* dxq, void* dsrc, void* ddest, void* fwd_state, void* ws, size_t ws_bytes, ua_stream_t stream);
+
+/* The same with every tensor described by its strides; dO: any rows; dkc, dvc (same strides) and dxq: row t at
+ * t * stride_inner. */
+int ua_fused_bwd_strided(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_rows* xq, const ua_gates* gates,
+                         const ua_rows* O, const float* lse, const ua_rows* dO, const ua_rows* dkc, const ua_rows* dvc,
+                         const ua_rows* dxq, const ua_gates* dgates, void* fwd_state, void* ws, size_t ws_bytes, ua_stream_t stream);
 
 /* Chunk merge: replaces SMVecMatMul.forward / .backward (universal_attention_autograd.py:278-297).
  * rows = number of (b,h,r,t) rows, n chunks, d features.  mat element (row, dd, i) at

@@ -21,6 +21,7 @@ UA_FLAG_RECOMPUTE = 4
 UA_FLAG_PRUNE = 2
 UA_FLAG_SHARE_GROUPS = 8
 UA_FLAG_GATES_F32 = 16
+UA_FLAG_FORWARD_ONLY = 32
 
 c_void_p, c_int, c_size_t, c_int64, c_int32 = ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t, ctypes.c_int64, ctypes.c_int32
 
@@ -31,6 +32,10 @@ class UaDesc(ctypes.Structure):
 
 class UaRows(ctypes.Structure):
     _fields_ = [("ptr", c_void_p)] + [(n, c_int64) for n in ("stride_b", "stride_h", "stride_r", "stride_outer", "stride_inner")] + [("inner_len", c_int32)]
+
+
+class UaGates(ctypes.Structure):
+    _fields_ = [("src", c_void_p), ("dest", c_void_p)] + [(n, c_int64) for n in ("stride_b", "stride_h", "stride_t")]
 
 
 class UaChunked(ctypes.Structure):
@@ -49,6 +54,9 @@ SIGNATURES = {
     "ua_bwd": (c_int, [P(UaDesc), P(UaRows), P(UaRows), P(UaRows), c_void_p, c_void_p, P(UaChunked), P(UaChunked), c_void_p,
                        c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "ua_fused_fwd": (c_int, [P(UaDesc), P(UaRows), P(UaRows), P(UaRows), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
+    "ua_fused_fwd_strided": (c_int, [P(UaDesc), P(UaRows), P(UaRows), P(UaRows), P(UaGates), P(UaRows), c_void_p, c_void_p, c_size_t, c_void_p]),
+    "ua_fused_bwd_strided": (c_int, [P(UaDesc), P(UaRows), P(UaRows), P(UaRows), P(UaGates), P(UaRows), c_void_p, P(UaRows), P(UaRows), P(UaRows),
+                                     P(UaRows), P(UaGates), c_void_p, c_void_p, c_size_t, c_void_p]),
     "ua_noalloc_scratch_bytes": (c_size_t, []),
     "ua_fused_fwd_noalloc": (c_int, [P(UaDesc), P(UaRows), P(UaRows), P(UaRows), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "ua_fused_bwd": (c_int, [P(UaDesc), P(UaRows), P(UaRows), P(UaRows), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
@@ -105,6 +113,28 @@ def load():
         from . import tune
         tune.load(env_file)
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The host module (csrc/ua_host.cpp: the differentiable entry points without Python between their kernels)."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _ua_host
+        except ImportError as e:
+            raise UaError("the host module _ua_host.so is missing or does not load (%s): build it with "
+                          "`python -m universal_attention_triton_amd.build`" % e)
+        if _ua_host.source_hash() != _lib.ua_source_hash().decode() and os.environ.get("UA_ALLOW_STALE_LIB") != "1":
+            raise UaError("_ua_host.so and libua_hip.so were built from different sources: rebuild them with "
+                          "`python -m universal_attention_triton_amd.build`")
+        from . import ops
+        _ua_host.init(UaError, ops)
+        _host = _ua_host
+    return _host
 
 
 def check(code, what):

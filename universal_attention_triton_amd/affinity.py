@@ -7,10 +7,15 @@ additive mask (reference _debug.py:123-164).
 """
 from torch.autograd import Function
 
-from . import ops
+from . import _lib, ops
 
 
 class AffinityScores(Function):
+    @classmethod
+    def apply(cls, k, src, dest):
+        aff = _lib.host().bias(k, src, dest)
+        return super().apply(k, src, dest) if aff is None else aff
+
     @staticmethod
     def forward(k, src, dest):
         return ops.affinity_forward(k, src, dest)

@@ -23,7 +23,7 @@ namespace ua {
 
 template <class T>
 struct BwdArgs {
-  const int *reach, *minkey;    // pruning state of the fused mode: [Zk][Lp/16], [Zk][Lp/32]
+  const int* reach;             // last query block every key tile reaches: [Zk][Lp/16]
   const int* masked_nz;         // chunked mode: non-zero when an upstream gradient of a (query, later chunk) pair is non-zero
   const T *Kp, *Vp;             // [Zk][Lp][D]
   const T *KT;                  // [Zk][D][Lp]
@@ -47,10 +47,11 @@ struct BwdArgs {
   int key_parts;                // k_bwd_keys2: sweeps per kv head (1 .. R, a divisor of R); dKrow, dVrow, dsrc_raw and dG_st hold one slice per (kv head, part)
   // direct (tile exchange, r = 1): the two kernels write the caller's gradients themselves and k_bwd_finish is not run:
   // k_bwd_keys2 dv and dsrc, k_bwd_queries3 dk (row side from dKrow + its own column side) and ddest.
-  // dk_out, dv_out [Z][L][d_out]; dsrc_out, ddest_out and the caller's gates src_in, dest_in [Z][L].
+  // dq_out (rows q_rows), dk_out and dv_out (rows kv_rows): the caller's tensors; gates: the caller's gates, dg: their gradients.
   int direct, d_out;
-  T *dk_out, *dv_out, *dsrc_out, *ddest_out;
-  const T *src_in, *dest_in;
+  T *dq_out, *dk_out, *dv_out;
+  RowsOut q_rows, kv_rows;
+  GateView gates, dg;
   // chunked operator with tile exchange: dOp is not the packed copy but the caller's upstream gradient itself, stored
   // chunk-major as rows of exactly D elements, [Zq*nch][L][D] with L a multiple of 32 (k_bwd_keys2 gathers its tiles)
   int dO_rows;
@@ -282,54 +283,53 @@ __global__ void __launch_bounds__(64 * NW) k_bwd_keys(BwdArgs<T> a) {
   }
 }
 
-// Combine partial gradients into the caller's contiguous tensors:
-//   dk [Zk][L][d], dv [Zk][L][d], dq [Zq][L][d], dsrc [Zk][L], ddest [Zk][L]
-// grid (ceil(L/4), max(Zk, Zq)); one wave per row.  The fp32 partial gradients are row-major [Z][Lp][D].
-// TG: dtype of the gates and of their gradients (the reference allocates dstatic_src in static_src.dtype,
-// Universal_Attention/triton/universal_attention_kernel.py:828)
-template <class T, class TG = T>
-__global__ void __launch_bounds__(256) k_bwd_finish(const float* __restrict__ dKrow, const float* __restrict__ dVrow,
-                                                    const float* __restrict__ dKdacc, const float* __restrict__ dQacc,
-                                                    const float* __restrict__ dsrc_raw, const T* __restrict__ Kp,
-                                                    const TG* __restrict__ src, const TG* __restrict__ dest,
-                                                    T* __restrict__ dk, T* __restrict__ dv, T* __restrict__ dq,
-                                                    TG* __restrict__ dsrc, TG* __restrict__ ddest, int Zk, int Zq, int L,
-                                                    int Lp, int D, int d, int tiled, int RS, int RK) {
-  const int z = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int t = blockIdx.x * 4 + wave;
-  if (t >= L) return;
-  if (z < Zq && dQacc) {
-    for (int c = lane; c < d; c += 64) dq[((long)z * L + t) * d + c] = cvt<T>(dQacc[((long)z * Lp + t) * D + c]);
-  }
-  if (z < Zk) {
-    const float sd = (float)dest[(long)z * L + t];
-    float dot = 0.f;
-    for (int c = lane; c < d; c += 64) {
-      const long i = ((long)z * Lp + t) * D + c;
-      // RS > 1: the column side comes in one slice per query group of the head
-      float kd = 0.f;
-      for (int r = 0; r < RS; ++r) kd += dKdacc[(((long)z * RS + r) * Lp + t) * D + c];
-      // the packed keys are row-major in chunked mode and tiled (nat_off) in fused mode
-      const long ik = !tiled ? i : (D == 64 ? nat_off<64>(z, Lp, t, c) : (D == 128 ? nat_off<128>(z, Lp, t, c) : nat_off<256>(z, Lp, t, c)));
-      dot += kd * (float)Kp[ik];
-      // RK > 1: so does the row side, and dV
-      float kr = 0.f, vr = 0.f;
-      for (int r = 0; r < RK; ++r) {
-        const long ir = (((long)z * RK + r) * Lp + t) * D + c;
-        kr += dKrow[ir];
-        vr += dVrow[ir];
-      }
-      dk[((long)z * L + t) * d + c] = cvt<T>(kr + kd);
-      dv[((long)z * L + t) * d + c] = cvt<T>(vr);
-    }
+// Combine partial gradients into the caller's tensors: dk, dv [Zk][L][d], the gate gradients [Zk][L] and, where dQ was summed
+// through atomics (dQacc), dq [Zq][L][d].  The fp32 partial gradients are row-major [Z][Lp][D], RS slices of the column side
+// and RK of the row side and of dV per kv head.  tiled: layout of the packed keys (nat_off instead of row-major).
+// grid (ceil(L / (1024 / D)), dQacc ? max(Zk, Zq) : Zk), 256 threads: D / 4 lanes per row, 16-byte loads.
+template <class T, int D>
+__global__ void __launch_bounds__(256) k_bwd_finish(BwdArgs<T> a, int Zk, int Zq, int tiled, int RS, int RK) {
+  constexpr int LPR = D / 4;
+  const int z = blockIdx.y, sub = threadIdx.x & (LPR - 1), c = 4 * sub, L = a.L, Lp = a.Lp, d = a.d_out;
+  const int t = blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+  if (t >= L) return;                       // all lanes of a row leave together
+  auto put4 = [&](T* p, const float (&x)[4]) {
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) dot += __shfl_xor(dot, m, 64);
-    if (lane == 0) {
-      ddest[(long)z * L + t] = cvt<TG>(dot / (2.0f * sd));
-      float sr = 0.f;
-      for (int r = 0; r < RK; ++r) sr += dsrc_raw[((long)z * RK + r) * Lp + t];
-      dsrc[(long)z * L + t] = cvt<TG>(sr / (3.0f * (float)src[(long)z * L + t]));
-    }
+    for (int e = 0; e < 4; ++e)
+      if (c + e < d) p[c + e] = cvt<T>(x[e]);
+  };
+  auto add4 = [&](const float* p, float (&x)[4]) {
+    const float4 v = *reinterpret_cast<const float4*>(p);
+    x[0] += v.x; x[1] += v.y; x[2] += v.z; x[3] += v.w;
+  };
+  if (a.dQacc && z < Zq) {
+    float q[4] = {0.f, 0.f, 0.f, 0.f};
+    add4(a.dQacc + ((long)z * Lp + t) * D + c, q);
+    put4(a.dq_out + rows_out(a.q_rows, z) + t * a.q_rows.st, q);
+  }
+  if (z >= Zk) return;
+  float kd[4] = {0.f, 0.f, 0.f, 0.f}, kr[4] = {0.f, 0.f, 0.f, 0.f}, vr[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int r = 0; r < RS; ++r) add4(a.dKdacc + (((long)z * RS + r) * Lp + t) * D + c, kd);
+  for (int r = 0; r < RK; ++r) {
+    const long o = (((long)z * RK + r) * Lp + t) * D + c;
+    add4(a.dKrow + o, kr);
+    add4(a.dVrow + o, vr);
+  }
+  const T* kp = a.Kp + (tiled ? nat_off<D>(z, Lp, t, c) : ((long)z * Lp + t) * D + c);      // 4 features of one cell either way
+  float dot = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) { dot += kd[e] * (float)kp[e]; kr[e] += kd[e]; }
+#pragma unroll
+  for (int m = LPR / 2; m >= 1; m >>= 1) dot += __shfl_xor(dot, m, 64);
+  const long row = rows_out(a.kv_rows, z) + t * a.kv_rows.st;
+  put4(a.dk_out + row, kr);
+  put4(a.dv_out + row, vr);
+  if (sub == 0) {
+    const long gi = gate_off(a.gates, z, t), go = gate_off(a.dg, z, t);
+    gate_put<T>(a.dg.dest, go, a.dg.f32, dot / (2.0f * gate_at<T>(a.gates.dest, gi, a.gates.f32)));
+    float sr = 0.f;
+    for (int r = 0; r < RK; ++r) sr += a.dsrc_raw[((long)z * RK + r) * Lp + t];
+    gate_put<T>(a.dg.src, go, a.dg.f32, sr / (3.0f * gate_at<T>(a.gates.src, gi, a.gates.f32)));
   }
 }
 

@@ -16,6 +16,7 @@
 #include "ua_merge.hpp"
 #include "ua_pack.hpp"
 #include "ua_bwd.hpp"   // k_bwd_finish only (k_bwd_keys is instantiated in ua_inst_bwd.hip)
+#include "ua_bwd_args.hpp"
 
 namespace {
 
@@ -35,7 +36,7 @@ struct Layout {
   int D, Lp, nT, nch, Zk, Zq;
   size_t esz;
   // forward state
-  size_t Kp, KT, Vp, VT, Qp, QT, lsrc, ldest, C, lse2, knorm2, qnorm2, reach, minkey, Bt, fwd_end;
+  size_t Kp, KT, Vp, VT, Qp, QT, lsrc, ldest, C, lse2, knorm2, qnorm2, reach, Bt, fwd_end;
   // backward scratch
   size_t dOp, dOT, delta, dQacc, dKdacc, Dsuf, dKrow, dVrow, dsrc_raw, masked_nz, dS_st, dG_st, total;
   bool tiles;       // bf16 merged operator: bias, dS and dG tiles are exchanged through the workspace
@@ -182,9 +183,8 @@ Layout make_layout(const ua_desc& d, bool chunked, int force_parts = 0) {
   l.lsrc = take((size_t)l.Zk * l.Lp * 4); l.ldest = take((size_t)l.Zk * l.Lp * 4);
   const size_t carries = (size_t)l.Zk * l.nT * l.Lp * 4;     // one float per (16-query tile, key)
   l.lse2 = take((size_t)l.Zq * l.nch * l.Lp * 4);
-  // pruning state of the fused mode: largest squared row norm of every 32-row block of K and Q, reach of every key
-  // tile, first key tile reaching every query block
-  l.knorm2 = take((size_t)l.Zk * (l.nT / 2) * 4); l.qnorm2 = take((size_t)l.Zq * (l.nT / 2) * 4); l.reach = take((size_t)l.Zk * l.nT * 4); l.minkey = take((size_t)l.Zk * (l.nT / 2) * 4);
+  // pruning state of the fused mode: largest squared row norm of every 32-row block of K and Q, reach of every key tile
+  l.knorm2 = take((size_t)l.Zk * (l.nT / 2) * 4); l.qnorm2 = take((size_t)l.Zq * (l.nT / 2) * 4); l.reach = take((size_t)l.Zk * l.nT * 4);
   // bf16 fused operator: the kernels exchange tiles through the workspace instead of recomputing them (fp16 bias of every
   // (16 keys, 32 queries) tile here; score and decay gradients in the backward part), 1 KB per tile
   l.tiles = !chunked && d.dtype == UA_BF16 && !(d.flags & UA_FLAG_RECOMPUTE);
@@ -231,13 +231,6 @@ ua::RowsView rows_view(const ua_rows& r, int H, int R) {
   v.H = H; v.R = R; v.N = 1;
   return v;
 }
-// contiguous [Z][L] (gates, lse) or [Z][L][d]
-ua::RowsView contiguous_view(const void* p, long z_stride, long row_stride) {
-  ua::RowsView v;
-  v.p = p; v.sb = z_stride; v.sh = 0; v.sr = 0; v.sn = 0; v.so = 0; v.si = row_stride; v.sc = 1;
-  v.inner = 1 << 30; v.H = 1; v.R = 1; v.N = 1;
-  return v;
-}
 // chunked tensor (zq, t, dd, i) seen as rows of z = zq*nch + i
 ua::RowsView chunked_view(const ua_chunked& c, int nch) {
   ua::RowsView v;
@@ -245,7 +238,6 @@ ua::RowsView chunked_view(const ua_chunked& c, int nch) {
   v.inner = 1 << 30; v.H = 1; v.R = 1; v.N = nch;
   return v;
 }
-ua::RowsView null_view() { ua::RowsView v{}; v.inner = 1; v.H = v.R = v.N = 1; return v; }
 
 // tr_mode: column order of the transposed copy inside each group of 32 positions
 enum { TR_PERM16 = 0, TR_PERM32 = 1, TR_NATURAL = 2 };
@@ -256,23 +248,39 @@ bool vector_ok(const ua::RowsView& v, size_t esz, int d) {
   return v.sc == 1 && d % V == 0 && (uintptr_t)v.p % 16 == 0 && al(v.sb) && al(v.sh) && al(v.sr) && al(v.sn) && al(v.so) && al(v.si);
 }
 template <class T>
-hipError_t pack_t(int D, const ua::RowsView& x, void* nat, void* tr, int d, int L, int Lp, int Z, int tr_mode, float* norm2,
-                  hipStream_t s, const int* masked_nz, int c) {
+hipError_t pack_t(int D, const ua::RowsView& x, void* nat, void* tr, int d, int L, int Lp, int Z, int tr_mode, hipStream_t s,
+                  const int* masked_nz, int c) {
   const int tiled = tr_mode != TR_PERM16;      // the fused kernels read tiled working tensors, the chunked ones row-major
   const int vec = vector_ok(x, sizeof(T), d) ? 1 : 0;
-  if (D == 256) {
-    if constexpr (sizeof(T) == 2) hipLaunchKernelGGL((ua::k_pack<T, 256>), dim3(Lp / 32, Z), dim3(256), 0, s, x, (T*)nat, (T*)tr, d, L, Lp, tr_mode, tiled, vec, norm2, masked_nz, c);
-    else return hipErrorInvalidValue;
-  } else if (D == 64) hipLaunchKernelGGL((ua::k_pack<T, 64>), dim3(Lp / 32, Z), dim3(256), 0, s, x, (T*)nat, (T*)tr, d, L, Lp, tr_mode, tiled, vec, norm2, masked_nz, c);
-  else hipLaunchKernelGGL((ua::k_pack<T, 128>), dim3(Lp / 32, Z), dim3(256), 0, s, x, (T*)nat, (T*)tr, d, L, Lp, tr_mode, tiled, vec, norm2, masked_nz, c);
+  if (D == 64) hipLaunchKernelGGL((ua::k_pack<T, 64>), dim3(Lp / 32, Z), dim3(256), 0, s, x, (T*)nat, (T*)tr, d, L, Lp, tr_mode, tiled, vec, masked_nz, c);
+  else hipLaunchKernelGGL((ua::k_pack<T, 128>), dim3(Lp / 32, Z), dim3(256), 0, s, x, (T*)nat, (T*)tr, d, L, Lp, tr_mode, tiled, vec, masked_nz, c);
   return hipGetLastError();
 }
-// norm2 (optional): [Z][Lp/32] receives the largest squared row norm of every block of 32 rows
-// masked_nz, c (optional, chunked upstream gradient): see k_pack
+// one tensor (head dims up to 128); masked_nz, c (optional, chunked upstream gradient): see k_pack
 hipError_t pack(int dtype, int D, const ua::RowsView& x, void* nat, void* tr, int d, int L, int Lp, int Z, int tr_mode, hipStream_t s,
-                float* norm2 = nullptr, const int* masked_nz = nullptr, int c = 0) {
-  return dtype == UA_BF16 ? pack_t<ua::bf16>(D, x, nat, tr, d, L, Lp, Z, tr_mode, norm2, s, masked_nz, c)
-                          : pack_t<float>(D, x, nat, tr, d, L, Lp, Z, tr_mode, norm2, s, masked_nz, c);
+                const int* masked_nz = nullptr, int c = 0) {
+  return dtype == UA_BF16 ? pack_t<ua::bf16>(D, x, nat, tr, d, L, Lp, Z, tr_mode, s, masked_nz, c)
+                          : pack_t<float>(D, x, nat, tr, d, L, Lp, Z, tr_mode, s, masked_nz, c);
+}
+ua::PackSrc pack_src(const ua::RowsView& v, int dtype, int d) { return ua::PackSrc{v, vector_ok(v, dtype == UA_BF16 ? 2 : 4, d) ? 1 : 0}; }
+template <class T, int D>
+hipError_t pack_inputs_t(const ua::PackInputs& p, long blocks, hipStream_t s) {
+  hipLaunchKernelGGL((ua::k_pack_inputs<T, D>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+  return hipGetLastError();
+}
+// heads: 2 Zk + Zq, or Zk for the keys and gates alone
+hipError_t launch_pack_inputs(int dtype, int D, const ua::PackInputs& p, int heads, hipStream_t s) {
+  const long blocks = (long)(p.Lp / 32) * heads;
+  if (dtype == UA_BF16) return D == 64 ? pack_inputs_t<ua::bf16, 64>(p, blocks, s) : D == 128 ? pack_inputs_t<ua::bf16, 128>(p, blocks, s) : pack_inputs_t<ua::bf16, 256>(p, blocks, s);
+  return D == 64 ? pack_inputs_t<float, 64>(p, blocks, s) : pack_inputs_t<float, 128>(p, blocks, s);
+}
+// dO -> working tensors and delta = dO . O of the merged operator
+template <class T, int D>
+hipError_t pack_grad_t(const ua::RowsView& dO, const ua::RowsView& O, const float* lse, void* nat, void* tr, float* delta, float* lse2,
+                       int d, int L, int Lp, int Z, hipStream_t s) {
+  hipLaunchKernelGGL((ua::k_pack_grad<T, D>), dim3((unsigned)((long)(Lp / 32) * Z)), dim3(256), 0, s, pack_src(dO, sizeof(T) == 2 ? UA_BF16 : UA_F32, d),
+                     pack_src(O, sizeof(T) == 2 ? UA_BF16 : UA_F32, d), lse, (T*)nat, (T*)tr, delta, lse2, d, L, Lp);
+  return hipGetLastError();
 }
 
 // ---- optional per-kernel timing (hipEvents on the launch stream) ---------------------------
@@ -339,45 +347,56 @@ bool gates_f32(const ua_desc& d) { return d.dtype == UA_F32 || (d.flags & UA_FLA
 // chunk sizes the query-stationary kernels handle (the others go through the key-chunk-stationary ones)
 bool fast_chunk(const ua_desc& d) { return d.chunk % 64 == 0; }
 
+ua::GateView gate_view(const ua_desc& d, const ua_gates& g) {
+  return ua::GateView{(void*)g.src, (void*)g.dest, (long)g.stride_b, (long)g.stride_h, (long)g.stride_t, d.h, gates_f32(d) ? 1 : 0};
+}
+ua_gates contiguous_gates(const ua_desc& d, const void* src, const void* dest) {
+  return ua_gates{(void*)src, (void*)dest, (int64_t)d.h * d.L, d.L, 1};
+}
+ua::RowsOut rows_out_of(const ua_desc& d, const ua_rows& r, int R) { return ua::RowsOut{(long)r.stride_b, (long)r.stride_h, (long)r.stride_r, (long)r.stride_inner, d.h, R}; }
+// contiguous [b, h, R, L, d]
+ua_rows contiguous_rows(const ua_desc& d, const void* p, int R) {
+  const int64_t head = (int64_t)d.L * d.d;
+  return ua_rows{p, head * R * d.h, head * R, head, 0, d.d, d.L};
+}
+
 // rowmajor: working tensors for the key-chunk-stationary (32x32 tile) kernels; otherwise the tiled layout
 int pack_inputs(const ua_desc& d, const Layout& l, bool rowmajor, const ua_rows* kc, const ua_rows* vc, const ua_rows* xq,
-                const void* src, const void* dest, char* wf, hipStream_t s) {
-  const bool chunked = rowmajor;
+                const ua_gates& gates, char* wf, hipStream_t s) {
   UA_PROF("pack_inputs", s);
-  const ua::RowsView K = rows_view(*kc, d.h, 1), V = rows_view(*vc, d.h, 1), Q = rows_view(*xq, d.h, d.r);
+  const bool prune = !rowmajor && (d.flags & UA_FLAG_PRUNE);
+  // the transposed keys and the natural values are read by the backward only (the chunked operator's fill reads the latter too)
+  const bool fwd_only = (d.flags & UA_FLAG_FORWARD_ONLY) && !rowmajor && l.nch == 1;
+  ua::PackInputs p{};
+  p.K = pack_src(rows_view(*kc, d.h, 1), d.dtype, d.d); p.V = pack_src(rows_view(*vc, d.h, 1), d.dtype, d.d);
+  p.Q = pack_src(rows_view(*xq, d.h, d.r), d.dtype, d.d);
+  p.g = gate_view(d, gates);
+  p.Kp = wf + l.Kp; p.KT = fwd_only ? nullptr : wf + l.KT; p.Vp = fwd_only ? nullptr : wf + l.Vp; p.VT = wf + l.VT; p.Qp = wf + l.Qp;
+  p.QT = l.grad_tiles || fwd_only ? nullptr : wf + l.QT;
+  p.lsrc = (float*)(wf + l.lsrc); p.ldest = (float*)(wf + l.ldest);
+  p.knorm2 = prune ? (float*)(wf + l.knorm2) : nullptr; p.qnorm2 = prune ? (float*)(wf + l.qnorm2) : nullptr;
+  p.Zk = l.Zk; p.d = d.d; p.L = d.L; p.Lp = l.Lp; p.tiled = rowmajor ? 0 : 1;
   // the chunked kernels work on 32x32 tiles, the fused ones on 16x16 tiles (and read V^T in natural order)
-  const int mode = chunked ? TR_PERM16 : TR_PERM32;
-  const bool prune = !chunked && (d.flags & UA_FLAG_PRUNE);
-  UA_HIP(pack(d.dtype, l.D, K, wf + l.Kp, wf + l.KT, d.d, d.L, l.Lp, l.Zk, mode, s, prune ? (float*)(wf + l.knorm2) : nullptr));
-  UA_HIP(pack(d.dtype, l.D, V, wf + l.Vp, wf + l.VT, d.d, d.L, l.Lp, l.Zk, chunked ? TR_PERM16 : TR_NATURAL, s));
-  UA_HIP(pack(d.dtype, l.D, Q, wf + l.Qp, l.grad_tiles ? nullptr : wf + l.QT, d.d, d.L, l.Lp, l.Zq, mode, s,
-              prune ? (float*)(wf + l.qnorm2) : nullptr));
-  const dim3 grid((l.Lp + 255) / 256, l.Zk);
-  if (!gates_f32(d))
-    hipLaunchKernelGGL((ua::k_gates<ua::bf16>), grid, dim3(256), 0, s, (const ua::bf16*)src, (const ua::bf16*)dest,
-                       (float*)(wf + l.lsrc), (float*)(wf + l.ldest), d.L, l.Lp);
-  else
-    hipLaunchKernelGGL((ua::k_gates<float>), grid, dim3(256), 0, s, (const float*)src, (const float*)dest,
-                       (float*)(wf + l.lsrc), (float*)(wf + l.ldest), d.L, l.Lp);
-  UA_HIP(hipGetLastError());
+  p.mode = rowmajor ? TR_PERM16 : TR_PERM32; p.vmode = rowmajor ? TR_PERM16 : TR_NATURAL;
+  UA_HIP(launch_pack_inputs(d.dtype, l.D, p, 2 * l.Zk + l.Zq, s));
   return UA_OK;
 }
 
 int launch_carry_for(const ua_desc& d, const Layout& l, char* wf, int variant, hipStream_t s) {
   UA_HIP(ua::launch_carry(d.dtype, l.D, wf + l.Kp, (const float*)(wf + l.lsrc), (const float*)(wf + l.ldest),
                           (float*)(wf + l.C), l.Lp, l.Zk, 1, (d.flags & UA_FLAG_PRUNE) ? (const float*)(wf + l.knorm2) : nullptr,
-                          (const float*)(wf + l.qnorm2), d.r, (int*)(wf + l.reach), (int*)(wf + l.minkey), s,
+                          (const float*)(wf + l.qnorm2), d.r, (int*)(wf + l.reach), s,
                           l.tiles ? wf + l.Bt : nullptr, variant));
   return UA_OK;
 }
-int launch_fwd_for(const ua_desc& d, const Layout& l, char* wf, void* O, float* lse, int variant, hipStream_t s) {
+int launch_fwd_for(const ua_desc& d, const Layout& l, char* wf, const ua_rows& O, float* lse, int variant, hipStream_t s) {
   UA_HIP(ua::launch_fwd_fused(d.dtype, l.D, variant, wf + l.Qp, wf + l.Kp, wf + l.VT, (const float*)(wf + l.lsrc),
-                              (const float*)(wf + l.ldest), (const float*)(wf + l.C), O, lse, (float*)(wf + l.lse2),
-                              (const int*)(wf + l.reach), (const int*)(wf + l.minkey), d.r, d.L, l.Lp, d.d, l.Zq, s,
+                              (const float*)(wf + l.ldest), (const float*)(wf + l.C), (void*)O.ptr, lse, (float*)(wf + l.lse2),
+                              (const int*)(wf + l.reach), d.r, d.L, l.Lp, d.d, l.Zq, rows_out_of(d, O, d.r), s,
                               l.tiles ? wf + l.Bt : nullptr));
   return UA_OK;
 }
-int run_fused_fwd_kernels(const ua_desc& d, const Layout& l, char* wf, void* O, float* lse, hipStream_t s) {
+int run_fused_fwd_kernels(const ua_desc& d, const Layout& l, char* wf, const ua_rows& O, float* lse, hipStream_t s) {
   {
     UA_PROF("k_carry", s);
     if (int e = launch_carry_for(d, l, wf, l.tiles ? tuned_variant(d, UA_TUNE_CARRY) : 0, s)) return e;
@@ -386,31 +405,38 @@ int run_fused_fwd_kernels(const ua_desc& d, const Layout& l, char* wf, void* O, 
   return launch_fwd_for(d, l, wf, O, lse, tuned_variant(d, l.tiles ? UA_TUNE_FWD_TILES : UA_TUNE_FWD_RECOMPUTE), s);
 }
 
-template <class T, class TG>
-hipError_t finish_t(const Layout& l, const ua_desc& d, char* wf, char* wb, bool chunked, const void* src, const void* dest, void* dk,
-                    void* dv, void* dq, void* dsrc, void* ddest, hipStream_t s) {
-  const int Z = l.Zq > l.Zk ? l.Zq : l.Zk;
-  hipLaunchKernelGGL((ua::k_bwd_finish<T, TG>), dim3((d.L + 3) / 4, Z), dim3(256), 0, s, (const float*)(wb + l.dKrow),
-                     (const float*)(wb + l.dVrow), (const float*)(wb + l.dKdacc), chunked ? (const float*)(wb + l.dQacc) : nullptr,
-                     (const float*)(wb + l.dsrc_raw), (const T*)(wf + l.Kp), (const TG*)src, (const TG*)dest, (T*)dk, (T*)dv,
-                     (T*)dq, (TG*)dsrc, (TG*)ddest, l.Zk, l.Zq, d.L, l.Lp, l.D, d.d, chunked ? 0 : 1, chunked ? 1 : d.r,
-                     l.key_parts);
+template <class T, int D>
+hipError_t finish_d(const ua::BwdArgsV& v, const Layout& l, bool atomics, hipStream_t s) {
+  ua::BwdArgs<T> a = ua::typed<T>(v);
+  if (!atomics) a.dQacc = nullptr;
+  constexpr int rows = 1024 / D;
+  hipLaunchKernelGGL((ua::k_bwd_finish<T, D>), dim3((v.L + rows - 1) / rows, atomics ? l.Zq : l.Zk), dim3(256), 0, s, a, l.Zk, l.Zq,
+                     atomics ? 0 : 1, atomics ? 1 : v.R, l.key_parts);
   return hipGetLastError();
+}
+hipError_t launch_finish(int dtype, const ua::BwdArgsV& v, const Layout& l, bool atomics, hipStream_t s) {
+  if (dtype == UA_BF16) return l.D == 64 ? finish_d<ua::bf16, 64>(v, l, atomics, s) : l.D == 128 ? finish_d<ua::bf16, 128>(v, l, atomics, s) : finish_d<ua::bf16, 256>(v, l, atomics, s);
+  return l.D == 64 ? finish_d<float, 64>(v, l, atomics, s) : finish_d<float, 128>(v, l, atomics, s);
 }
 
 template <class T>
-hipError_t delta_t(const ua::RowsView& O, const ua::RowsView& dO, const ua::RowsView& sub, const ua::RowsView& lse_in,
-                   float* delta, float* lse2, int d, int L, int Lp, int Z, hipStream_t s, int* masked_nz = nullptr, int c = 0) {
+hipError_t delta_t(const ua::RowsView& O, const ua::RowsView& dO, const ua::RowsView& sub, float* delta, int d, int L, int Lp, int Z,
+                   hipStream_t s, int* masked_nz = nullptr, int c = 0) {
   const int vec = vector_ok(O, sizeof(T), d) && vector_ok(dO, sizeof(T), d) ? 1 : 0;
-  hipLaunchKernelGGL((ua::k_delta<T>), dim3(Lp / 128, Z), dim3(256), 0, s, O, dO, sub, lse_in, delta, lse2, d, L, Lp, vec, masked_nz, c);
+  hipLaunchKernelGGL((ua::k_delta<T>), dim3(Lp / 128, Z), dim3(256), 0, s, O, dO, sub, delta, d, L, Lp, vec, masked_nz, c);
   return hipGetLastError();
 }
 
+// where a backward leaves its results
+struct GradOut {
+  ua_rows dk, dv, dq;      // dk and dv share their strides
+  ua_gates gates, dgates;
+};
+
 // chunked with a chunk that is not a multiple of 64: key-chunk-stationary kernel over row-major working tensors (atomics);
 // otherwise the key-stationary and query-stationary kernels over tiled working tensors
-int run_bwd_common(const ua_desc& d, const Layout& l, char* wf, char* wb, bool chunked, const void* src, const void* dest, void* dkc,
-                   void* dvc, void* dxq, void* dsrc, void* ddest, hipStream_t s, const float* delta_given = nullptr,
-                   const float* lse2_given = nullptr, const void* dO_rows = nullptr) {
+int run_bwd_common(const ua_desc& d, const Layout& l, char* wf, char* wb, bool chunked, const GradOut& out, hipStream_t s,
+                   const float* delta_given = nullptr, const float* lse2_given = nullptr, const void* dO_rows = nullptr) {
   const bool is_chunked = chunked;
   chunked = is_chunked && !fast_chunk(d);      // from here on: the atomics path
   if (chunked) {
@@ -422,7 +448,7 @@ int run_bwd_common(const ua_desc& d, const Layout& l, char* wf, char* wb, bool c
   a.Kp = wf + l.Kp; a.Vp = wf + l.Vp; a.KT = wf + l.KT; a.Qp = wf + l.Qp; a.QT = l.grad_tiles ? nullptr : wf + l.QT; a.dOp = wb + l.dOp;
   a.dOT = l.grad_tiles ? nullptr : wb + l.dOT; a.lsrc = (const float*)(wf + l.lsrc); a.ldest = (const float*)(wf + l.ldest);
   a.lse2 = lse2_given ? lse2_given : (const float*)(wf + l.lse2); a.delta = delta_given ? delta_given : (const float*)(wb + l.delta); a.C = (const float*)(wf + l.C);
-  a.reach = (const int*)(wf + l.reach); a.minkey = (const int*)(wf + l.minkey);
+  a.reach = (const int*)(wf + l.reach);
   a.dQacc = (float*)(wb + l.dQacc); a.dKdacc = (float*)(wb + l.dKdacc); a.Dsuf = (float*)(wb + l.Dsuf);
   a.dKrow = (float*)(wb + l.dKrow);
   a.dVrow = (float*)(wb + l.dVrow); a.dsrc_raw = (float*)(wb + l.dsrc_raw);
@@ -439,9 +465,11 @@ int run_bwd_common(const ua_desc& d, const Layout& l, char* wf, char* wb, bool c
   // operator qualifies when the caller asserts that nothing flows to (query, later chunk) pairs, so that the query side is
   // known here to run from the tiles.
   const bool from_tiles = l.tiles || (is_chunked && l.grad_tiles && (d.flags & UA_FLAG_SKIP_MASKED));
-  const bool direct = from_tiles && d.r == 1 && !gates_f32(d);
-  a.direct = direct ? 1 : 0; a.d_out = d.d; a.dk_out = dkc; a.dv_out = dvc; a.dsrc_out = dsrc; a.ddest_out = ddest;
-  a.src_in = src; a.dest_in = dest;
+  const bool direct = from_tiles && d.r == 1;
+  a.direct = direct ? 1 : 0; a.d_out = d.d;
+  a.dq_out = (void*)out.dq.ptr; a.dk_out = (void*)out.dk.ptr; a.dv_out = (void*)out.dv.ptr;
+  a.q_rows = rows_out_of(d, out.dq, d.r); a.kv_rows = rows_out_of(d, out.dk, 1);
+  a.gates = gate_view(d, out.gates); a.dg = gate_view(d, out.dgates);
   {
     UA_PROF("k_bwd_keys", s);
     UA_HIP(ua::launch_bwd_keys(d.dtype, l.D, a, l.Zk, chunked ? 1 : 0, s));
@@ -449,14 +477,12 @@ int run_bwd_common(const ua_desc& d, const Layout& l, char* wf, char* wb, bool c
   if (!chunked) {
     UA_PROF("k_bwd_queries", s);
     // chunked operator with tiles: both are enqueued, the flag k_delta left on the device decides which one works
-    if (l.grad_tiles) UA_HIP(ua::launch_bwd_queries_from_tiles(l.D, a, dxq, d.d, l.Zq, s, tuned_variant(d, UA_TUNE_BWD_QUERIES)));
-    if (!from_tiles) UA_HIP(ua::launch_bwd_queries(d.dtype, l.D, a, dxq, d.d, l.Zk, s));
+    if (l.grad_tiles) UA_HIP(ua::launch_bwd_queries_from_tiles(l.D, a, d.d, l.Zq, s, tuned_variant(d, UA_TUNE_BWD_QUERIES)));
+    if (!from_tiles) UA_HIP(ua::launch_bwd_queries(d.dtype, l.D, a, d.d, l.Zk, s));
   }
   if (direct) return UA_OK;
   UA_PROF("k_bwd_finish", s);
-  if (d.dtype == UA_BF16 && gates_f32(d)) UA_HIP((finish_t<ua::bf16, float>(l, d, wf, wb, chunked, src, dest, dkc, dvc, dxq, dsrc, ddest, s)));
-  else if (d.dtype == UA_BF16) UA_HIP((finish_t<ua::bf16, ua::bf16>(l, d, wf, wb, chunked, src, dest, dkc, dvc, dxq, dsrc, ddest, s)));
-  else UA_HIP((finish_t<float, float>(l, d, wf, wb, chunked, src, dest, dkc, dvc, dxq, dsrc, ddest, s)));
+  UA_HIP(launch_finish(d.dtype, a, l, chunked, s));
   return UA_OK;
 }
 
@@ -520,16 +546,24 @@ size_t ua_workspace_bytes(const ua_desc* desc, int op) {
   return l.total;
 }
 
+int ua_fused_fwd_strided(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_rows* xq, const ua_gates* gates,
+                         const ua_rows* O, float* lse, void* ws, size_t ws_bytes, ua_stream_t stream) {
+  if (int e = check_desc(desc, false)) return e;
+  const Layout l = make_layout(*desc, false);
+  if (!gates) return fail(UA_EINVAL, "null gates");
+  if (int e = check_common(kc, vc, xq, gates->src, gates->dest, ws, ws_bytes, l.fwd_end)) return e;
+  if (!O || !O->ptr || !lse) return fail(UA_EINVAL, "null output tensor");
+  char* wf = (char*)ws;
+  hipStream_t s = (hipStream_t)stream;
+  if (int e = pack_inputs(*desc, l, false, kc, vc, xq, *gates, wf, s)) return e;
+  return run_fused_fwd_kernels(*desc, l, wf, *O, lse, s);
+}
 int ua_fused_fwd(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_rows* xq, const void* static_src,
                  const void* static_dest, void* O, float* lse, void* ws, size_t ws_bytes, ua_stream_t stream) {
   if (int e = check_desc(desc, false)) return e;
-  const Layout l = make_layout(*desc, false);
-  if (int e = check_common(kc, vc, xq, static_src, static_dest, ws, ws_bytes, l.fwd_end)) return e;
-  if (!O || !lse) return fail(UA_EINVAL, "null output tensor");
-  char* wf = (char*)ws;
-  hipStream_t s = (hipStream_t)stream;
-  if (int e = pack_inputs(*desc, l, false, kc, vc, xq, static_src, static_dest, wf, s)) return e;
-  return run_fused_fwd_kernels(*desc, l, wf, O, lse, s);
+  const ua_gates g = contiguous_gates(*desc, static_src, static_dest);
+  const ua_rows o = contiguous_rows(*desc, O, desc->r);
+  return ua_fused_fwd_strided(desc, kc, vc, xq, &g, &o, lse, ws, ws_bytes, stream);
 }
 
 // ---- forward for callers that cannot allocate: scratch in a device array of the library itself ----------------
@@ -572,31 +606,42 @@ int ua_fused_fwd_noalloc(const ua_desc* desc, const ua_rows* kc, const ua_rows* 
   return ua_fused_fwd(desc, kc, vc, xq, static_src, static_dest, O, lse, ws, UA_NOALLOC_SCRATCH_BYTES, stream);
 }
 
-int ua_fused_bwd(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_rows* xq, const void* static_src,
-                 const void* static_dest, const void* O, const float* lse, const void* dO, void* dkc, void* dvc, void* dxq,
-                 void* dsrc, void* ddest, void* fwd_state, void* ws, size_t ws_bytes, ua_stream_t stream) {
+int ua_fused_bwd_strided(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_rows* xq, const ua_gates* gates,
+                         const ua_rows* O, const float* lse, const ua_rows* dO, const ua_rows* dkc, const ua_rows* dvc,
+                         const ua_rows* dxq, const ua_gates* dgates, void* fwd_state, void* ws, size_t ws_bytes, ua_stream_t stream) {
   if (int e = check_desc(desc, false)) return e;
   const Layout l = make_layout(*desc, false);
-  if (int e = check_common(kc, vc, xq, static_src, static_dest, ws, ws_bytes, fwd_state ? l.total - l.fwd_end : l.total)) return e;
-  if (!O || !lse || !dO || !dkc || !dvc || !dxq || !dsrc || !ddest) return fail(UA_EINVAL, "null tensor");
+  if (!gates || !dgates || !O || !dO || !dkc || !dvc || !dxq) return fail(UA_EINVAL, "null tensor");
+  if (int e = check_common(kc, vc, xq, gates->src, gates->dest, ws, ws_bytes, fwd_state ? l.total - l.fwd_end : l.total)) return e;
+  if (!O->ptr || !lse || !dO->ptr || !dkc->ptr || !dvc->ptr || !dxq->ptr || !dgates->src || !dgates->dest) return fail(UA_EINVAL, "null tensor");
+  if (dkc->stride_b != dvc->stride_b || dkc->stride_h != dvc->stride_h || dkc->stride_inner != dvc->stride_inner)
+    return fail(UA_EINVAL, "dkc and dvc must have the same strides");
   char *wf, *wb;
   if (int e = bwd_bases(l, fwd_state, ws, &wf, &wb)) return e;
   hipStream_t s = (hipStream_t)stream;
   const ua_desc& d = *desc;
   if (!fwd_state) {
-    if (int e = pack_inputs(d, l, false, kc, vc, xq, static_src, static_dest, wf, s)) return e;
+    if (int e = pack_inputs(d, l, false, kc, vc, xq, *gates, wf, s)) return e;
     if (int e = launch_carry_for(d, l, wf, l.tiles ? tuned_variant(d, UA_TUNE_CARRY) : 0, s)) return e;
   }
-  const long rowsz = (long)d.L * d.d;
-  const ua::RowsView Ov = contiguous_view(O, rowsz, d.d), dOv = contiguous_view(dO, rowsz, d.d);
-  const ua::RowsView lsev = contiguous_view(lse, d.L, 1), none = null_view();
   {
     UA_PROF("pack_dO+delta", s);
-    UA_HIP(pack(d.dtype, l.D, dOv, wb + l.dOp, l.grad_tiles ? nullptr : wb + l.dOT, d.d, d.L, l.Lp, l.Zq, TR_PERM32, s));
-    if (d.dtype == UA_BF16) UA_HIP(delta_t<ua::bf16>(Ov, dOv, none, lsev, (float*)(wb + l.delta), (float*)(wf + l.lse2), d.d, d.L, l.Lp, l.Zq, s));
-    else UA_HIP(delta_t<float>(Ov, dOv, none, lsev, (float*)(wb + l.delta), (float*)(wf + l.lse2), d.d, d.L, l.Lp, l.Zq, s));
+#define UA_PG(T, D_) UA_HIP((pack_grad_t<T, D_>(rows_view(*dO, d.h, d.r), rows_view(*O, d.h, d.r), lse, wb + l.dOp,   \
+                                                l.grad_tiles ? nullptr : wb + l.dOT, (float*)(wb + l.delta), (float*)(wf + l.lse2), d.d, d.L, l.Lp, l.Zq, s)))
+    if (d.dtype == UA_BF16) { if (l.D == 64) UA_PG(ua::bf16, 64); else if (l.D == 128) UA_PG(ua::bf16, 128); else UA_PG(ua::bf16, 256); }
+    else { if (l.D == 64) UA_PG(float, 64); else UA_PG(float, 128); }
+#undef UA_PG
   }
-  return run_bwd_common(d, l, wf, wb, false, static_src, static_dest, dkc, dvc, dxq, dsrc, ddest, s);
+  return run_bwd_common(d, l, wf, wb, false, GradOut{*dkc, *dvc, *dxq, *gates, *dgates}, s);
+}
+int ua_fused_bwd(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_rows* xq, const void* static_src,
+                 const void* static_dest, const void* O, const float* lse, const void* dO, void* dkc, void* dvc, void* dxq,
+                 void* dsrc, void* ddest, void* fwd_state, void* ws, size_t ws_bytes, ua_stream_t stream) {
+  if (int e = check_desc(desc, false)) return e;
+  const ua_gates g = contiguous_gates(*desc, static_src, static_dest), dg = contiguous_gates(*desc, dsrc, ddest);
+  const ua_rows o = contiguous_rows(*desc, O, desc->r), go = contiguous_rows(*desc, dO, desc->r), dk = contiguous_rows(*desc, dkc, 1),
+                dv = contiguous_rows(*desc, dvc, 1), dq = contiguous_rows(*desc, dxq, desc->r);
+  return ua_fused_bwd_strided(desc, kc, vc, xq, &g, &o, lse, &go, &dk, &dv, &dq, &dg, fwd_state, ws, ws_bytes, stream);
 }
 
 int ua_fwd(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_rows* xq, const void* static_src,
@@ -609,6 +654,7 @@ int ua_fwd(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_r
   char* wf = (char*)ws;
   hipStream_t s = (hipStream_t)stream;
   const ua_desc& d = *desc;
+  const ua_gates gates = contiguous_gates(d, static_src, static_dest);
   float* lse2 = lse2_out ? lse2_out : (float*)(wf + l.lse2);     // the per-chunk normalisers, float32, log2 units
   // the workspace stays a complete forward state for ua_bwd also when the normalisers went to the caller's buffer
   auto mirror_lse2 = [&]() -> int {
@@ -616,21 +662,21 @@ int ua_fwd(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_r
     return UA_OK;
   };
   if (fast_chunk(d)) {
-    if (int e = pack_inputs(d, l, false, kc, vc, xq, static_src, static_dest, wf, s)) return e;
+    if (int e = pack_inputs(d, l, false, kc, vc, xq, gates, wf, s)) return e;
     {
       UA_PROF("k_carry", s);
       UA_HIP(ua::launch_carry(d.dtype, l.D, wf + l.Kp, (const float*)(wf + l.lsrc), (const float*)(wf + l.ldest), (float*)(wf + l.C), l.Lp,
-                              l.Zk, 1, nullptr, nullptr, d.r, (int*)(wf + l.reach), (int*)(wf + l.minkey), s));
+                              l.Zk, 1, nullptr, nullptr, d.r, (int*)(wf + l.reach), s));
     }
     UA_PROF("k_fwd_chunked", s);
     UA_HIP(ua::launch_fwd_chunked2(d.dtype, l.D, wf + l.Qp, wf + l.Kp, wf + l.Vp, wf + l.VT, (const float*)(wf + l.lsrc),
                                    (const float*)(wf + l.ldest), (const float*)(wf + l.C), (const int*)(wf + l.reach),
-                                   (const int*)(wf + l.minkey), out->ptr, denom, lse2, out->stride_z, out->stride_t,
+                                   out->ptr, denom, lse2, out->stride_z, out->stride_t,
                                    out->stride_d, out->stride_i, d.r, d.L, l.Lp, d.d, d.chunk, l.nch, l.Zq, s,
                                    tuned_variant(d, UA_TUNE_CHUNKED_PAIR)));
     return mirror_lse2();
   }
-  if (int e = pack_inputs(d, l, true, kc, vc, xq, static_src, static_dest, wf, s)) return e;
+  if (int e = pack_inputs(d, l, true, kc, vc, xq, gates, wf, s)) return e;
   UA_PROF("k_fwd_chunked", s);
   UA_HIP(ua::launch_fwd_chunked(d.dtype, l.D, wf + l.Qp, wf + l.Kp, wf + l.VT, (const float*)(wf + l.lsrc),
                                 (const float*)(wf + l.ldest), out->ptr, denom, lse2, out->stride_z, out->stride_t, out->stride_d, out->stride_i, d.r, d.L,
@@ -652,9 +698,11 @@ int ua_bwd(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_r
   if (int e = bwd_bases(l, fwd_state, ws, &wf, &wb)) return e;
   hipStream_t s = (hipStream_t)stream;
   const ua_desc& d = *desc;
+  const ua_gates gates = contiguous_gates(d, static_src, static_dest);
+  const GradOut grads{contiguous_rows(d, dkc, 1), contiguous_rows(d, dvc, 1), contiguous_rows(d, dxq, d.r), gates, contiguous_gates(d, dsrc, ddest)};
   const ua::RowsView outv = chunked_view(*out, l.nch);
   ua_chunked gmut = *g_out;
-  const ua::RowsView gv = chunked_view(gmut, l.nch), none = null_view();
+  const ua::RowsView gv = chunked_view(gmut, l.nch);
   // g_denom [zq][t][i] seen per z = zq*nch + i
   ua::RowsView gdv;
   gdv.p = g_denom; gdv.sb = (long)d.L * l.nch; gdv.sh = 0; gdv.sr = 0; gdv.sn = 1; gdv.so = 0; gdv.si = l.nch; gdv.sc = 1;
@@ -662,13 +710,13 @@ int ua_bwd(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_r
   if (fast_chunk(d)) {
     if (!fwd_state) {
       // recompute the carries and the per-chunk normalisers (the partial outputs themselves are passed in)
-      if (int e = pack_inputs(d, l, false, kc, vc, xq, static_src, static_dest, wf, s)) return e;
+      if (int e = pack_inputs(d, l, false, kc, vc, xq, gates, wf, s)) return e;
       UA_HIP(ua::launch_carry(d.dtype, l.D, wf + l.Kp, (const float*)(wf + l.lsrc), (const float*)(wf + l.ldest), (float*)(wf + l.C), l.Lp,
-                              l.Zk, 1, nullptr, nullptr, d.r, (int*)(wf + l.reach), (int*)(wf + l.minkey), s));
+                              l.Zk, 1, nullptr, nullptr, d.r, (int*)(wf + l.reach), s));
       if (!lse2_in)
         UA_HIP(ua::launch_fwd_chunked2(d.dtype, l.D, wf + l.Qp, wf + l.Kp, wf + l.Vp, wf + l.VT, (const float*)(wf + l.lsrc),
                                        (const float*)(wf + l.ldest), (const float*)(wf + l.C), (const int*)(wf + l.reach),
-                                       (const int*)(wf + l.minkey), nullptr, nullptr, (float*)(wf + l.lse2), 0, 0, 0, 0, d.r, d.L, l.Lp,
+                                       nullptr, nullptr, (float*)(wf + l.lse2), 0, 0, 0, 0, d.r, d.L, l.Lp,
                                        d.d, d.chunk, l.nch, l.Zq, s, tuned_variant(d, UA_TUNE_CHUNKED_PAIR)));
     }
     bool in_place = false;
@@ -679,8 +727,8 @@ int ua_bwd(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_r
       int* nz = (int*)(wb + l.masked_nz);
       int* detect = (d.flags & UA_FLAG_SKIP_MASKED) ? nullptr : nz;
       if (delta) { /* ua_merge_bwd left it: neither out nor g_out is read for it */ }
-      else if (d.dtype == UA_BF16) UA_HIP(delta_t<ua::bf16>(outv, gv, gdv, none, (float*)(wb + l.delta), nullptr, d.d, d.L, l.Lp, l.Zq * l.nch, s, detect, d.chunk));
-      else UA_HIP(delta_t<float>(outv, gv, gdv, none, (float*)(wb + l.delta), nullptr, d.d, d.L, l.Lp, l.Zq * l.nch, s, detect, d.chunk));
+      else if (d.dtype == UA_BF16) UA_HIP(delta_t<ua::bf16>(outv, gv, gdv, (float*)(wb + l.delta), d.d, d.L, l.Lp, l.Zq * l.nch, s, detect, d.chunk));
+      else UA_HIP(delta_t<float>(outv, gv, gdv, (float*)(wb + l.delta), d.d, d.L, l.Lp, l.Zq * l.nch, s, detect, d.chunk));
       // With the tile exchange only the key-side kernel reads the upstream gradient, and when nothing flows to the
       // (query, later chunk) pairs (UA_FLAG_SKIP_MASKED) it can gather its tiles from the caller's tensor itself if that
       // is stored chunk-major in rows of exactly D elements: no packed copy (half of g_out read, as much written).
@@ -688,26 +736,26 @@ int ua_bwd(const ua_desc* desc, const ua_rows* kc, const ua_rows* vc, const ua_r
                  g_out->stride_t == d.d && g_out->stride_i == (int64_t)d.L * d.d && g_out->stride_z == (int64_t)l.nch * d.L * d.d &&
                  (uintptr_t)g_out->ptr % 16 == 0;
       if (!in_place)
-        UA_HIP(pack(d.dtype, l.D, gv, wb + l.dOp, l.grad_tiles ? nullptr : wb + l.dOT, d.d, d.L, l.Lp, l.Zq * l.nch, TR_PERM32, s, nullptr, nz,
+        UA_HIP(pack(d.dtype, l.D, gv, wb + l.dOp, l.grad_tiles ? nullptr : wb + l.dOT, d.d, d.L, l.Lp, l.Zq * l.nch, TR_PERM32, s, nz,
                     d.chunk));
     }
-    return run_bwd_common(d, l, wf, wb, true, static_src, static_dest, dkc, dvc, dxq, dsrc, ddest, s, delta, lse2_in,
+    return run_bwd_common(d, l, wf, wb, true, grads, s, delta, lse2_in,
                           in_place ? g_out->ptr : nullptr);
   }
   if (delta) return fail(UA_EINVAL, "a precomputed delta needs UA_FLAG_SKIP_MASKED and a chunk that is a multiple of 64");
   if (!fwd_state) {
     // recompute the per-chunk normalisers (the partial outputs themselves are passed in)
-    if (int e = pack_inputs(d, l, true, kc, vc, xq, static_src, static_dest, wf, s)) return e;
+    if (int e = pack_inputs(d, l, true, kc, vc, xq, gates, wf, s)) return e;
     if (!lse2_in)
       UA_HIP(ua::launch_fwd_chunked(d.dtype, l.D, wf + l.Qp, wf + l.Kp, wf + l.VT, (const float*)(wf + l.lsrc),
                                     (const float*)(wf + l.ldest), nullptr, nullptr, (float*)(wf + l.lse2), 0, 0, 0, 0, d.r, d.L, l.Lp, d.d, d.chunk, l.nch, l.Zk, s));
   }
   UA_HIP(ua::launch_carry(d.dtype, l.D, wf + l.Kp, (const float*)(wf + l.lsrc), (const float*)(wf + l.ldest),
-                          (float*)(wf + l.C), l.Lp, l.Zk, 0, nullptr, nullptr, 1, nullptr, nullptr, s));
+                          (float*)(wf + l.C), l.Lp, l.Zk, 0, nullptr, nullptr, 1, nullptr, s));
   UA_HIP(pack(d.dtype, l.D, gv, wb + l.dOp, wb + l.dOT, d.d, d.L, l.Lp, l.Zq * l.nch, TR_PERM16, s));
-  if (d.dtype == UA_BF16) UA_HIP(delta_t<ua::bf16>(outv, gv, gdv, none, (float*)(wb + l.delta), nullptr, d.d, d.L, l.Lp, l.Zq * l.nch, s));
-  else UA_HIP(delta_t<float>(outv, gv, gdv, none, (float*)(wb + l.delta), nullptr, d.d, d.L, l.Lp, l.Zq * l.nch, s));
-  return run_bwd_common(d, l, wf, wb, true, static_src, static_dest, dkc, dvc, dxq, dsrc, ddest, s, nullptr, lse2_in);
+  if (d.dtype == UA_BF16) UA_HIP(delta_t<ua::bf16>(outv, gv, gdv, (float*)(wb + l.delta), d.d, d.L, l.Lp, l.Zq * l.nch, s));
+  else UA_HIP(delta_t<float>(outv, gv, gdv, (float*)(wb + l.delta), d.d, d.L, l.Lp, l.Zq * l.nch, s));
+  return run_bwd_common(d, l, wf, wb, true, grads, s, nullptr, lse2_in);
 }
 
 // 16-byte accesses to every (row, chunk) slice of a chunked tensor, with d / V lanes per slice (a power of two <= 64)
@@ -794,16 +842,13 @@ int aff_prepare(const ua_desc* desc, const ua_rows* k, const void* src, const vo
   if (ws_bytes < need) return fail(UA_EWORKSPACE, "workspace has %zu bytes, %zu needed", ws_bytes, need);
   const ua_desc& d = *desc;
   char* w = (char*)ws;
-  const ua::RowsView K = rows_view(*k, d.h, 1);
-  UA_HIP(pack(d.dtype, l.D, K, w + l.Kp, w + l.KT, d.d, d.L, l.Lp, l.Z, TR_PERM32, s));
-  const dim3 grid((l.Lp + 255) / 256, l.Z);
-  if (d.dtype == UA_BF16)
-    hipLaunchKernelGGL((ua::k_gates<ua::bf16>), grid, dim3(256), 0, s, (const ua::bf16*)src, (const ua::bf16*)dest,
-                       (float*)(w + l.lsrc), (float*)(w + l.ldest), d.L, l.Lp);
-  else
-    hipLaunchKernelGGL((ua::k_gates<float>), grid, dim3(256), 0, s, (const float*)src, (const float*)dest,
-                       (float*)(w + l.lsrc), (float*)(w + l.ldest), d.L, l.Lp);
-  UA_HIP(hipGetLastError());
+  ua::PackInputs p{};
+  p.K = pack_src(rows_view(*k, d.h, 1), d.dtype, d.d);
+  p.g = gate_view(d, contiguous_gates(d, src, dest));
+  p.g.f32 = d.dtype == UA_F32;
+  p.Kp = w + l.Kp; p.KT = bwd ? w + l.KT : nullptr; p.lsrc = (float*)(w + l.lsrc); p.ldest = (float*)(w + l.ldest);
+  p.Zk = l.Z; p.d = d.d; p.L = d.L; p.Lp = l.Lp; p.tiled = 1; p.mode = TR_PERM32;
+  UA_HIP(launch_pack_inputs(d.dtype, l.D, p, l.Z, s));      // keys and gates only
   return UA_OK;
 }
 }  // namespace
@@ -903,11 +948,11 @@ int ua_autotune(const ua_desc* desc, int op, void* ws, size_t ws_bytes, ua_strea
     void* Otmp = wb + l.dOp;                  // [Zq][L][d] fits in [Zq][Lp][D]
     float* lsetmp = (float*)(wb + l.delta);
     if (l.tiles) {
-      if (int e = tune_slot(d, UA_TUNE_FWD_TILES, s, [&](int v) { return launch_fwd_for(d, l, w, Otmp, lsetmp, v, s); })) return e;
+      if (int e = tune_slot(d, UA_TUNE_FWD_TILES, s, [&](int v) { return launch_fwd_for(d, l, w, contiguous_rows(d, Otmp, d.r), lsetmp, v, s); })) return e;
       // the pre-pass rewrites the bias tiles, the reach table and the first-key table with the same values
       if (int e = tune_slot(d, UA_TUNE_CARRY, s, [&](int v) { return launch_carry_for(d, l, w, v, s); })) return e;
     } else {
-      if (int e = tune_slot(d, UA_TUNE_FWD_RECOMPUTE, s, [&](int v) { return launch_fwd_for(d, l, w, Otmp, lsetmp, v, s); })) return e;
+      if (int e = tune_slot(d, UA_TUNE_FWD_RECOMPUTE, s, [&](int v) { return launch_fwd_for(d, l, w, contiguous_rows(d, Otmp, d.r), lsetmp, v, s); })) return e;
     }
     return UA_OK;
   }
@@ -918,7 +963,7 @@ int ua_autotune(const ua_desc* desc, int op, void* ws, size_t ws_bytes, ua_strea
     a.Kp = wf + ll.Kp; a.Vp = wf + ll.Vp; a.KT = wf + ll.KT; a.Qp = wf + ll.Qp; a.dOp = wb + ll.dOp;
     a.lsrc = (const float*)(wf + ll.lsrc); a.ldest = (const float*)(wf + ll.ldest); a.lse2 = (const float*)(wf + ll.lse2);
     a.delta = (const float*)(wb + ll.delta); a.C = (const float*)(wf + ll.C);
-    a.reach = (const int*)(wf + ll.reach); a.minkey = (const int*)(wf + ll.minkey);
+    a.reach = (const int*)(wf + ll.reach);
     a.dKdacc = (float*)(wb + ll.dKdacc); a.dKrow = (float*)(wb + ll.dKrow); a.dVrow = (float*)(wb + ll.dVrow);
     a.dsrc_raw = (float*)(wb + ll.dsrc_raw); a.masked_nz = (const int*)(wb + ll.masked_nz);
     a.dS_st = wb + ll.dS_st; a.dG_st = wb + ll.dG_st; a.Bt = wf + ll.Bt;
@@ -926,10 +971,12 @@ int ua_autotune(const ua_desc* desc, int op, void* ws, size_t ws_bytes, ua_strea
     // one query group: the production path has both kernels write the caller's gradients from their epilogues and runs no
     // finish pass, so the slots are timed that way, with throw-away outputs in the scratch (dv over the dV partial sums,
     // dk over the column-side partial sums, the gate gradients over the dsrc partial sums; "gates" read from the log-gates)
-    if (d.r == 1 && !gates_f32(d)) {
+    a.q_rows = rows_out_of(d, contiguous_rows(d, nullptr, d.r), d.r); a.kv_rows = rows_out_of(d, contiguous_rows(d, nullptr, 1), 1);
+    if (d.r == 1) {
       a.direct = 1; a.d_out = d.d;
-      a.dv_out = wb + ll.dVrow; a.dk_out = wb + ll.dKdacc; a.dsrc_out = wb + ll.dsrc_raw; a.ddest_out = wb + ll.dsrc_raw;
-      a.src_in = wf + ll.lsrc; a.dest_in = wf + ll.ldest;
+      a.dv_out = wb + ll.dVrow; a.dk_out = wb + ll.dKdacc;
+      a.gates = gate_view(d, contiguous_gates(d, wf + ll.lsrc, wf + ll.ldest));
+      a.dg = gate_view(d, contiguous_gates(d, wb + ll.dsrc_raw, wb + ll.dsrc_raw));
     }
     return a;
   };
@@ -957,10 +1004,10 @@ int ua_autotune(const ua_desc* desc, int op, void* ws, size_t ws_bytes, ua_strea
         })) return e;
   }
   {
-    const ua::BwdArgsV a = bwd_args(l);
-    void* dqtmp = wb + l.dOp;
+    ua::BwdArgsV a = bwd_args(l);
+    a.dq_out = wb + l.dOp;
     if (int e = tune_slot(d, UA_TUNE_BWD_QUERIES, s, [&](int v) {
-          UA_HIP(ua::launch_bwd_queries_from_tiles(l.D, a, dqtmp, d.d, l.Zq, s, v));
+          UA_HIP(ua::launch_bwd_queries_from_tiles(l.D, a, d.d, l.Zq, s, v));
           return (int)UA_OK;
         })) return e;
   }

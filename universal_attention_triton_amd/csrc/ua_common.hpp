@@ -19,6 +19,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "ua_views.hpp"
 
 namespace ua {
 
@@ -224,6 +225,45 @@ __device__ __forceinline__ void xcd_map(int& bx, int& by) {
     by = (n & 7) + 8 * (slot / gx);
     bx = slot % gx;
   }
+}
+__device__ __forceinline__ long rows_out(const RowsOut& o, int z) {
+  return (long)(z / (o.H * o.R)) * o.sb + (long)(z / o.R % o.H) * o.sh + (long)(z % o.R) * o.sr;
+}
+__device__ __forceinline__ long gate_off(const GateView& g, int z, int t) { return (long)(z / g.H) * g.sb + (long)(z % g.H) * g.sh + (long)t * g.st; }
+template <class T> __device__ __forceinline__ float gate_at(const void* p, long off, int f32) {
+  return f32 ? reinterpret_cast<const float*>(p)[off] : (float)reinterpret_cast<const T*>(p)[off];
+}
+template <class T> __device__ __forceinline__ void gate_put(void* p, long off, int f32, float x) {
+  if (f32) reinterpret_cast<float*>(p)[off] = x;
+  else reinterpret_cast<T*>(p)[off] = cvt<T>(x);
+}
+// The kernel's first argument, read again from the argument segment: for what only an epilogue needs.  Taken from the
+// parameter itself it is loaded at the start and held over the sweep, where scalar registers are short (k_bwd_keys2: 38 spilled
+// instead of 13, 2.52 instead of 2.29 ms at b = 1, h = 32, L = 8192, d = 128).
+template <class A> __device__ __forceinline__ const A& late_args() {
+  unsigned long long p = (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *reinterpret_cast<const A*>(p);
+}
+// First key tile (of 16) that reaches query block tb: reach_z[sb] >= tb (tiles 2 tb and 2 tb + 1 hold the block's own
+// keys).  Every wave looks it up for itself, 512 tiles per round trip; without pruning the first tile is a hit.
+__device__ __forceinline__ int first_key_tile(const int* __restrict__ reach_z, int tb, int lane) {
+  for (int sb0 = 0; sb0 < 2 * tb; sb0 += 512) {
+    const int sb = sb0 + 8 * lane;
+    int first = 8;
+    if (sb < 2 * tb) {         // reach has a multiple of 8 entries per head
+      const int4 x = *reinterpret_cast<const int4*>(reach_z + sb), y = *reinterpret_cast<const int4*>(reach_z + sb + 4);
+      const int r[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+      for (int e = 7; e >= 0; --e) first = r[e] >= tb ? e : first;
+    }
+    const unsigned long long hit = __builtin_amdgcn_ballot_w64(first < 8);
+    if (hit) {
+      const int l = __builtin_ctzll(hit);
+      return min(sb0 + 8 * l + __builtin_amdgcn_readlane(first, l), 2 * tb);
+    }
+  }
+  return 2 * tb;
 }
 // CUs of the current device (launchers choose between one and two work items per workgroup by it)
 inline int device_cus() {

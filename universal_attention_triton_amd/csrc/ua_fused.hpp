@@ -241,16 +241,6 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
   }
 }
 
-// minkey[z][tb] = first key tile (of 16) that reaches query block tb; it never decreases with tb.
-template <class Unused = void>
-__global__ void __launch_bounds__(256) k_minkey(const int* __restrict__ reach, int* __restrict__ minkey, int nT16) {
-  const int z = blockIdx.y, tb = blockIdx.x * 256 + threadIdx.x, nT32 = nT16 / 2;
-  if (tb >= nT32) return;
-  int sb = 0;
-  while (sb < 2 * tb && reach[z * nT16 + sb] < tb) ++sb;          // tiles 2 tb and 2 tb + 1 hold the block's own keys
-  minkey[z * nT32 + tb] = sb;
-}
-
 // Destination of the per-chunk results of the chunked operator (reference universal_attention_autograd.py:9-38):
 // out element (zq, t, dd, i) at zq*sz + t*st + dd*sd + i*si, denom [Zq][L][nch]; either may be null.
 template <class T> struct ChunkOut {
@@ -351,11 +341,11 @@ __global__ void __launch_bounds__(256) k_chunk_masked_denom(T* __restrict__ deno
 // 32-query block share the block's key, value and bias tiles: the workgroup then covers 4 / RB blocks of RB heads
 // (grid (Lp / (128 / RB), Zk * R / RB)) instead of 4 blocks of one head.
 template <class T, int D, int NST, int NW, bool CHUNKED, bool BI = false, int RB = 1>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW >= 8 ? (BI && NST == 1 ? (D > 128 ? 2 : 4) : NW / 4) : (BI ? 3 : 2), NW >= 8 ? (BI && NST == 1 ? (D > 128 ? 2 : 4) : NW / 4) : (BI ? 3 : 2)))) k_fwd_fused2(const T* __restrict__ Qp, const T* __restrict__ Kp,
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW >= 8 ? (BI && NST == 1 ? (D > 128 ? 2 : 4) : NW / 4) : (BI ? 3 : 2), NW >= 8 ? (BI && NST == 1 ? (D > 128 ? 2 : 4) : NW / 4) : (BI ? 3 : 2)))) k_fwd_fused2(RowsOut orow_arg, const T* __restrict__ Qp, const T* __restrict__ Kp,
                                                     const T* __restrict__ VT, const float* __restrict__ lsrc,
                                                     const float* __restrict__ ldest, const float* __restrict__ C,
                                                     T* __restrict__ O, float* __restrict__ lse, float* __restrict__ lse2,
-                                                    const int* __restrict__ reach, const int* __restrict__ minkey,
+                                                    const int* __restrict__ reach,
                                                     int R, int L, int Lp, int d, ChunkOut<T> co,
                                                     const _Float16* __restrict__ Bt = nullptr) {
   static_assert(!BI || ((NW == 8 || NW == 4) && !CHUNKED), "bias tiles: 4 or 8 waves, merged operator");
@@ -413,7 +403,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
   // key tiles that cannot reach this workgroup's first query block (see k_carry2) are not visited at all; inside
   // the visited range a tile that does not reach this wave's block gets a carry of -1e30 (its weights become 0)
   const int tbq = tq >> 1;
-  const int kt_min = minkey[zk * (nT16 >> 1) + NB * jt] >> 2;
+  const int kt_min = first_key_tile(reach + zk * nT16, NB * jt, lane) >> 2;
   const int n_steps = n_kt - kt_min;
   // per-wave stats row of a step: [C row: 64f][lsrc: 64f][reach of the 4 key tiles: 4 ints]; source of each lane's
   // 16 bytes as base + step * stride (in 4-byte units)
@@ -602,6 +592,9 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
 #undef UA_COMPUTE_SLOW
   // epilogue
   if (CHUNKED || !live) return;
+  const RowsOut& orow = late_args<RowsOut>();
+  T* const O_z = O + rows_out(orow, zq);
+  const long o_st = orow.st;
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     const float tot = allsum16(ls[v]);
@@ -611,7 +604,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
 #pragma unroll
       for (int n = 0; n < ND; ++n) {
         const int dd = 16 * n + col;
-        if (dd < d) O[((long)zq * L + t) * d + dd] = cvt<T>(o[n][v] * inv);
+        if (dd < d) O_z[t * o_st + dd] = cvt<T>(o[n][v] * inv);
       }
     }
     if (col == 0) {
@@ -645,8 +638,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
 // ---------------------------------------------------------------------------------------------
 template <int D, int RB>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_fwd_fused3(const bf16* __restrict__ Qp, const bf16* __restrict__ Kp, const bf16* __restrict__ VT, bf16* __restrict__ O,
-             float* __restrict__ lse, float* __restrict__ lse2, const int* __restrict__ reach, const int* __restrict__ minkey,
+k_fwd_fused3(RowsOut orow_arg, const bf16* __restrict__ Qp, const bf16* __restrict__ Kp, const bf16* __restrict__ VT, bf16* __restrict__ O,
+             float* __restrict__ lse, float* __restrict__ lse2, const int* __restrict__ reach,
              int R, int L, int Lp, int d, const _Float16* __restrict__ Bt) {
   using T = bf16;
   using TN = Tile<T, 32, D>;
@@ -695,7 +688,7 @@ k_fwd_fused3(const bf16* __restrict__ Qp, const bf16* __restrict__ Kp, const bf1
   const int qb_end = min(NB * (jt + 1), nT32);
   const int n_kt = (qb_end + 1) / 2;                          // key tiles of 64 covering s <= last query of the workgroup
   // key tiles that cannot reach this workgroup's first query block (see k_carry2) are not visited
-  const int kt_min = minkey[zk * nT32 + NB * jt] >> 2;
+  const int kt_min = first_key_tile(reach + zk * nT16, NB * jt, lane) >> 2;
   const int n_steps = n_kt - kt_min;
   // this lane's 16 bytes of key tile 0 of the wave's query block
   const char* bt_src = reinterpret_cast<const char*>(Bt) + (((long)zk * tri_tiles(nT32) + tri_bias_row(qb)) << 10) + 16 * lane;
@@ -817,6 +810,9 @@ k_fwd_fused3(const bf16* __restrict__ Qp, const bf16* __restrict__ Kp, const bf1
 #undef UA_COMPUTE_FAST
 #undef UA_COMPUTE_SLOW
   if (!live) return;
+  const RowsOut& orow = late_args<RowsOut>();
+  T* const O_z = O + rows_out(orow, zq);
+  const long o_st = orow.st;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -828,7 +824,7 @@ k_fwd_fused3(const bf16* __restrict__ Qp, const bf16* __restrict__ Kp, const bf1
 #pragma unroll
         for (int n = 0; n < ND; ++n) {
           const int dd = 16 * n + col;
-          if (dd < d) O[((long)zq * L + t) * d + dd] = cvt<T>(o[i][n][v] * inv);
+          if (dd < d) O_z[t * o_st + dd] = cvt<T>(o[i][n][v] * inv);
         }
       }
       if (col == 0) {
@@ -1231,12 +1227,20 @@ __global__ void __launch_bounds__(512) k_bwd_keys2(BwdArgs<T> a) {
     float b, af, tot;
     group_scan(dsrc_acc, gm, b, af, tot);
     if (TO && !MR && a.direct) {      // straight into the caller's tensor: dsrc = sum dA A / (3 src)
-      if (g == 0 && spos < L) a.dsrc_out[(long)zo * L + spos] = cvt<T>(1.5f * tot / (3.0f * (float)a.src_in[(long)zo * L + spos]));
+      const BwdArgs<T>& e = late_args<BwdArgs<T>>();
+      if (g == 0 && spos < L) gate_put<T>(e.dg.src, gate_off(e.dg, zo, spos), e.dg.f32, 1.5f * tot / (3.0f * gate_at<T>(e.gates.src, gate_off(e.gates, zo, spos), e.gates.f32)));
     } else if (g == 0) {
       a.dsrc_raw[(long)zo * Lp + spos] = 1.5f * tot;    // sum dA A = 3/2 sum dG G
     }
   }
   const bool direct = TO && !MR && a.direct;
+  T* dv_row = nullptr;
+  int d_out = 0;
+  if (direct) {
+    const BwdArgs<T>& e = late_args<BwdArgs<T>>();
+    dv_row = e.dv_out + rows_out(e.kv_rows, zo) + spos * e.kv_rows.st;
+    d_out = e.d_out;
+  }
 #pragma unroll
   for (int n = 0; n < ND; ++n) {
     const long o = ((long)zo * Lp + spos) * D + 16 * n + 4 * g;
@@ -1244,10 +1248,10 @@ __global__ void __launch_bounds__(512) k_bwd_keys2(BwdArgs<T> a) {
     if (!direct) {
       *reinterpret_cast<float4*>(a.dVrow + o) = make_float4(dVt[n][0], dVt[n][1], dVt[n][2], dVt[n][3]);
     } else if (spos < L) {
-      T* dst = a.dv_out + ((long)zo * L + spos) * a.d_out + 16 * n + 4 * g;
+      T* dst = dv_row + 16 * n + 4 * g;
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        if (16 * n + 4 * g + v < a.d_out) dst[v] = cvt<T>(dVt[n][v]);
+        if (16 * n + 4 * g + v < d_out) dst[v] = cvt<T>(dVt[n][v]);
     }
   }
   };
@@ -1269,7 +1273,7 @@ __global__ void __launch_bounds__(512) k_bwd_keys2(BwdArgs<T> a) {
 // CH: chunked operator (a.c a multiple of 64): the upstream gradient, delta and the normaliser are those of the chunk
 // the step's 64 keys belong to (z index zq*nch + chunk) and are reloaded when the chunk changes.
 template <class T, int D, int NST, bool CH>
-__global__ void __launch_bounds__(512) k_bwd_queries2(BwdArgs<T> a, T* __restrict__ dq, int d) {
+__global__ void __launch_bounds__(512) k_bwd_queries2(BwdArgs<T> a, int d) {
   using TN = Tile<T, 32, D>;
   using TT = Tile<T, D, 32>;
   constexpr int NK = D / 32, ND = D / 16;
@@ -1316,7 +1320,7 @@ __global__ void __launch_bounds__(512) k_bwd_queries2(BwdArgs<T> a, T* __restric
   // key tiles out of reach of this workgroup's first query block are not visited (see k_carry2); inside the range
   // a tile that does not reach this wave's block gets a carry of -1e30, which zeroes its dS and dG
   const int tbq = tq >> 1;
-  const int kt_min = (a.minkey[zk * (nT16 >> 1) + 4 * jt] >> 2) & ~1;
+  const int kt_min = (first_key_tile(a.reach + zk * nT16, 4 * jt, lane) >> 2) & ~1;
   // per-wave stats row of a step: [C row: 64f][lsrc: 64f][Dsuf row: 64f][reach of the 4 key tiles: 4 ints] and, with
   // the chunked operator, [lse2: 16f][delta: 16f] of this wave's queries in the step's chunk at floats 208 and 224; source of
   // each lane's 16 bytes as base + step * stride (in 4-byte units)
@@ -1542,7 +1546,7 @@ __global__ void __launch_bounds__(512) k_bwd_queries2(BwdArgs<T> a, T* __restric
 #pragma unroll
         for (int n = 0; n < ND; ++n) {
           const int dd = 16 * n + col;
-          if (dd < d) dq[(zq * L + t) * d + dd] = cvt<T>(dQ[n][v]);
+          if (dd < d) a.dq_out[rows_out(a.q_rows, zq) + t * a.q_rows.st + dd] = cvt<T>(dQ[n][v]);
         }
       }
     }
@@ -1568,7 +1572,7 @@ __global__ void __launch_bounds__(512) k_bwd_queries2(BwdArgs<T> a, T* __restric
 // bytes: more of them in flight, and one workgroup's prologue and epilogue under the other's stream).
 template <class T, int D, int NST, int HV>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(HV == 1 ? 4 : 2, HV == 1 ? 4 : 2)))
-k_bwd_queries3(BwdArgs<T> a, T* __restrict__ dq, int d) {
+k_bwd_queries3(BwdArgs<T> a, int d) {
   static_assert(sizeof(T) == 2, "tiles are exchanged in 16-bit operand precision");
   static_assert(HV == 1 || HV == 2, "one or two key halves per step");
   using TT = Tile<T, D, 32>;
@@ -1594,7 +1598,7 @@ k_bwd_queries3(BwdArgs<T> a, T* __restrict__ dq, int d) {
   for (int n = 0; n < ND; ++n) { dQ[n] = (f32x4){0, 0, 0, 0}; dKc[n] = (f32x4){0, 0, 0, 0}; }
   const T* KTz = a.KT + (long)zk * D * Lp;
   const int n_kt = (4 * jt + 4) / HV;                  // steps of 32 HV keys
-  const int kt_min = (a.minkey[zk * (nT16 >> 1) + 4 * jt] >> (HV == 2 ? 2 : 1)) & ~1;
+  const int kt_min = (first_key_tile(a.reach + zk * nT16, 4 * jt, lane) >> (HV == 2 ? 2 : 1)) & ~1;
   // this lane's 16 bytes of the wave's tiles of key half h: base + h * 1024
   const long st_head = grp_tiles(Lp >> 5) << 10;
   const char* pS = reinterpret_cast<const char*>(a.dS_st) + (long)zq * st_head + (grp_tile(tq, 0) << 10) + 16 * lane;
@@ -1653,7 +1657,10 @@ k_bwd_queries3(BwdArgs<T> a, T* __restrict__ dq, int d) {
   constexpr int RS = 64 + 4;            // floats per staged row: the four row groups of a store hit different banks
   static_assert(4 * 16 * RS * 4 <= SB, "staging area");
   float* xs = reinterpret_cast<float*>((w < 4 ? stage0 : stage1) + (w & 3) * (16 * RS * 4));
-  const bool vec_ok = (d & 3) == 0 && ((reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(a.dk_out)) & 7) == 0;
+  const bool vec_ok = (d & 3) == 0 && ((reinterpret_cast<uintptr_t>(a.dq_out) | reinterpret_cast<uintptr_t>(a.dk_out)) & 7) == 0 &&
+                      ((a.q_rows.sb | a.q_rows.sh | a.q_rows.sr | a.q_rows.st | a.kv_rows.sb | a.kv_rows.sh | a.kv_rows.st) & 3) == 0;
+  T* const dq_z = a.dq_out + rows_out(a.q_rows, zq);
+  T* const dk_z = a.dk_out + rows_out(a.kv_rows, zk);
   auto stage_half = [&] __device__ (const f32x4 (&X)[ND], int hf, f32x4 (&out)[4]) {
 #pragma unroll
     for (int nn = 0; nn < 4; ++nn)
@@ -1664,18 +1671,18 @@ k_bwd_queries3(BwdArgs<T> a, T* __restrict__ dq, int d) {
     for (int i = 0; i < 4; ++i) out[i] = *reinterpret_cast<const f32x4*>(xs + (4 * i + g) * RS + 4 * col);
     __builtin_amdgcn_wave_barrier();
   };
-  auto store4 = [&] __device__ (T* dst, long row, int f0, const f32x4& x) {      // 4 consecutive features of a row of d
+  auto store4 = [&] __device__ (T* dst, int f0, const f32x4& x) {      // 4 consecutive features of a row
     if (vec_ok) {
       if (f0 < d) {
         union { T h[4]; u32x2 u; } pk;
 #pragma unroll
         for (int e = 0; e < 4; ++e) pk.h[e] = cvt<T>(x[e]);
-        __builtin_nontemporal_store(pk.u, reinterpret_cast<u32x2*>(dst + row * d + f0));
+        __builtin_nontemporal_store(pk.u, reinterpret_cast<u32x2*>(dst + f0));
       }
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (f0 + e < d) dst[row * d + f0 + e] = cvt<T>(x[e]);
+        if (f0 + e < d) dst[f0 + e] = cvt<T>(x[e]);
     }
   };
   float dot[4] = {0.f, 0.f, 0.f, 0.f};
@@ -1698,7 +1705,7 @@ k_bwd_queries3(BwdArgs<T> a, T* __restrict__ dq, int d) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int t = 16 * tq + 4 * i + g;
-      if (t < L) store4(dq, (long)zq * L + t, f0, x[i]);
+      if (t < L) store4(dq_z + t * a.q_rows.st, f0, x[i]);
     }
     stage_half(dKc, hf, x);
 #pragma unroll
@@ -1708,7 +1715,7 @@ k_bwd_queries3(BwdArgs<T> a, T* __restrict__ dq, int d) {
         const T* kk = reinterpret_cast<const T*>(&kraw[i]);
 #pragma unroll
         for (int e = 0; e < 4; ++e) dot[i] = __builtin_fmaf(x[i][e], (float)kk[e], dot[i]);      // padded features: k = 0
-        if (t < L) store4(a.dk_out, (long)zq * L + t, f0, x[i] + krow[i]);
+        if (t < L) store4(dk_z + t * a.kv_rows.st, f0, x[i] + krow[i]);
       } else {
         *reinterpret_cast<f32x4*>(a.dKdacc + ((long)zq * Lp + t) * D + f0) = x[i];
       }
@@ -1719,7 +1726,7 @@ k_bwd_queries3(BwdArgs<T> a, T* __restrict__ dq, int d) {
     for (int i = 0; i < 4; ++i) {
       const int t = 16 * tq + 4 * i + g;
       const float sum = allsum16(dot[i]);
-      if (col == 0 && t < L) a.ddest_out[(long)zq * L + t] = cvt<T>(sum / (2.0f * (float)a.dest_in[(long)zq * L + t]));
+      if (col == 0 && t < L) gate_put<T>(a.dg.dest, gate_off(a.dg, zq, t), a.dg.f32, sum / (2.0f * gate_at<T>(a.gates.dest, gate_off(a.gates, zq, t), a.gates.f32)));
     }
   }
   };

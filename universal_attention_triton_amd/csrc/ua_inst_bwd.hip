@@ -80,31 +80,31 @@ hipError_t launch_bwd_keys(int dtype, int D, const BwdArgsV& a, int Zk, int cols
 
 // explicit instantiations (the implicit ones are not emitted on the host side for this kernel)
 #define UA_INST(T, D, NST)                                                      \
-  template __global__ void k_bwd_queries2<T, D, NST, false>(BwdArgs<T>, T*, int); \
-  template __global__ void k_bwd_queries2<T, D, NST, true>(BwdArgs<T>, T*, int);
+  template __global__ void k_bwd_queries2<T, D, NST, false>(BwdArgs<T>, int); \
+  template __global__ void k_bwd_queries2<T, D, NST, true>(BwdArgs<T>, int);
 UA_INST(bf16, 64, 2) UA_INST(bf16, 128, 2) UA_INST(float, 64, 1) UA_INST(float, 128, 1)
 #undef UA_INST
 
 template <class T, int D, int NST>
-static hipError_t bwdq_t(const BwdArgsV& v, void* dq, int d, int Zk, hipStream_t s) {
+static hipError_t bwdq_t(const BwdArgsV& v, int d, int Zk, hipStream_t s) {
   const BwdArgs<T> a = typed<T>(v);
   const dim3 grid(v.Lp / 128, v.split_r ? Zk * v.R : Zk);
-  if (v.chunked) hipLaunchKernelGGL((k_bwd_queries2<T, D, NST, true>), grid, dim3(512), 0, s, a, (T*)dq, d);
-  else hipLaunchKernelGGL((k_bwd_queries2<T, D, NST, false>), grid, dim3(512), 0, s, a, (T*)dq, d);
+  if (v.chunked) hipLaunchKernelGGL((k_bwd_queries2<T, D, NST, true>), grid, dim3(512), 0, s, a, d);
+  else hipLaunchKernelGGL((k_bwd_queries2<T, D, NST, false>), grid, dim3(512), 0, s, a, d);
   return hipGetLastError();
 }
-hipError_t launch_bwd_queries(int dtype, int D, const BwdArgsV& a, void* dq, int d, int Zk, hipStream_t s) {
+hipError_t launch_bwd_queries(int dtype, int D, const BwdArgsV& a, int d, int Zk, hipStream_t s) {
   if (D == 256) return hipErrorInvalidValue;   // the recomputing query side stops at 128
-  if (dtype == 1) return D == 64 ? bwdq_t<bf16, 64, 2>(a, dq, d, Zk, s) : bwdq_t<bf16, 128, 2>(a, dq, d, Zk, s);
-  return D == 64 ? bwdq_t<float, 64, 1>(a, dq, d, Zk, s) : bwdq_t<float, 128, 1>(a, dq, d, Zk, s);
+  if (dtype == 1) return D == 64 ? bwdq_t<bf16, 64, 2>(a, d, Zk, s) : bwdq_t<bf16, 128, 2>(a, d, Zk, s);
+  return D == 64 ? bwdq_t<float, 64, 1>(a, d, Zk, s) : bwdq_t<float, 128, 1>(a, d, Zk, s);
 }
 
-template __global__ void k_bwd_queries3<bf16, 64, 2, 1>(BwdArgs<bf16>, bf16*, int);
-template __global__ void k_bwd_queries3<bf16, 128, 2, 1>(BwdArgs<bf16>, bf16*, int);
-template __global__ void k_bwd_queries3<bf16, 64, 2, 2>(BwdArgs<bf16>, bf16*, int);
-template __global__ void k_bwd_queries3<bf16, 256, 2, 1>(BwdArgs<bf16>, bf16*, int);
-template __global__ void k_bwd_queries3<bf16, 128, 2, 2>(BwdArgs<bf16>, bf16*, int);
-hipError_t launch_bwd_queries_from_tiles(int D, const BwdArgsV& v, void* dq, int d, int Zq, hipStream_t s, int variant) {
+template __global__ void k_bwd_queries3<bf16, 64, 2, 1>(BwdArgs<bf16>, int);
+template __global__ void k_bwd_queries3<bf16, 128, 2, 1>(BwdArgs<bf16>, int);
+template __global__ void k_bwd_queries3<bf16, 64, 2, 2>(BwdArgs<bf16>, int);
+template __global__ void k_bwd_queries3<bf16, 256, 2, 1>(BwdArgs<bf16>, int);
+template __global__ void k_bwd_queries3<bf16, 128, 2, 2>(BwdArgs<bf16>, int);
+hipError_t launch_bwd_queries_from_tiles(int D, const BwdArgsV& v, int d, int Zq, hipStream_t s, int variant) {
   const BwdArgs<bf16> a = typed<bf16>(v);
   // steps of 32 keys (two workgroups per CU): four query blocks per workgroup once every CU gets at least eight of the
   // single ones, two once it gets four; steps of 64 keys: one block per workgroup
@@ -115,7 +115,7 @@ hipError_t launch_bwd_queries_from_tiles(int D, const BwdArgsV& v, void* dq, int
                  : (n_blk % 4 == 0 && n_wg >= 8L * device_cus()) ? n_blk / 4
                  : n_wg >= 4L * device_cus() ? (n_blk + 1) / 2 : n_blk;
   const dim3 grid(gx, Zq);
-#define UA_Q3(D_, HV_) hipLaunchKernelGGL((k_bwd_queries3<bf16, D_, 2, HV_>), grid, dim3(512), 0, s, a, (bf16*)dq, d)
+#define UA_Q3(D_, HV_) hipLaunchKernelGGL((k_bwd_queries3<bf16, D_, 2, HV_>), grid, dim3(512), 0, s, a, d)
   if (D == 256) UA_Q3(256, 1);              // steps of 32 keys only: a stage of 64 keys would not fit twice
   else if (variant == 1) { if (D == 64) UA_Q3(64, 2); else UA_Q3(128, 2); }
   else { if (D == 64) UA_Q3(64, 1); else UA_Q3(128, 1); }

@@ -459,8 +459,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
   // epilogue
   const float tot = dsrc_acc + xor_lane(dsrc_acc, 32);
   const bool direct = a.direct;
+  T* dv_row = nullptr;
+  int d_out = 0;
   if (direct) {      // straight into the caller's tensor: dsrc = sum dA A / (3 src), sum dA A = 3/2 sum dG G
-    if (hi == 0 && spos < L) a.dsrc_out[(long)zo * L + spos] = cvt<T>(1.5f * tot / (3.0f * (float)a.src_in[(long)zo * L + spos]));
+    const BwdArgs<T>& e = late_args<BwdArgs<T>>();
+    dv_row = e.dv_out + rows_out(e.kv_rows, zo) + spos * e.kv_rows.st;
+    d_out = e.d_out;
+    if (hi == 0 && spos < L) gate_put<T>(e.dg.src, gate_off(e.dg, zo, spos), e.dg.f32, 1.5f * tot / (3.0f * gate_at<T>(e.gates.src, gate_off(e.gates, zo, spos), e.gates.f32)));
   } else if (hi == 0) {
     a.dsrc_raw[(long)zo * Lp + spos] = 1.5f * tot;
   }
@@ -474,10 +479,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
       if (!direct) {
         *reinterpret_cast<float4*>(a.dVrow + o) = make_float4(dVt[n][4 * g], dVt[n][4 * g + 1], dVt[n][4 * g + 2], dVt[n][4 * g + 3]);
       } else if (spos < L) {
-        T* dst = a.dv_out + ((long)zo * L + spos) * a.d_out + f0;
+        T* dst = dv_row + f0;
 #pragma unroll
         for (int v = 0; v < 4; ++v)
-          if (f0 + v < a.d_out) dst[v] = cvt<T>(dVt[n][4 * g + v]);
+          if (f0 + v < d_out) dst[v] = cvt<T>(dVt[n][4 * g + v]);
       }
     }
   }

@@ -12,6 +12,7 @@ dimension must have stride 1), so nothing is copied on the way in except the two
 """
 import torch
 
+from . import ops
 from .universal_attention import universal_attention
 
 
@@ -25,7 +26,7 @@ def split_gates(static, n_kv):
 
 def decoder_attention(query_state, key_state, value_state, static, chunk=128, prune=False, recompute=False):
     """query_state [b, s, n, d], key_state / value_state [b, s, n_kv, d], static [b, s, 2*n_kv] (gates in (0, 1))
-    -> attention output [b, s, n, d] (a permuted view of the operator's [b, n_kv, rep, s, d] result).
+    -> attention output [b, s, n, d].
 
     Query head j belongs to kv head j // rep (reference main.py:26: view(b, n_kv, rep, s, d)).  `chunk` only shapes the
     views the operator's interface asks for; the fused result does not depend on it.  Differentiable."""
@@ -33,6 +34,12 @@ def decoder_attention(query_state, key_state, value_state, static, chunk=128, pr
     n_kv = key_state.shape[2]
     assert key_state.shape == (b, s, n_kv, d) and value_state.shape == (b, s, n_kv, d)
     assert n % n_kv == 0, "query heads must be a multiple of kv heads"
+    host = ops.native()
+    if host is not None and not ops.tune_on_first_call():
+        # the tensors as they are, gates and their gradients included: no views, so no autograd node per view
+        res = host.decoder(query_state, key_state, value_state, static, prune, recompute)
+        if res is not None:
+            return res[0]
     rep = n // n_kv
     c = chunk if s % chunk == 0 else s
     xq = query_state.transpose(1, 2).unflatten(1, (n_kv, rep))          # [b, n_kv, rep, s, d], strided view

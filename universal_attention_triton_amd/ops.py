@@ -1,6 +1,7 @@
 """Host-side operators over the C ABI: tensor plumbing only (device memory, strides, streams)."""
 import ctypes
 import functools
+import os
 import weakref
 
 import torch
@@ -101,6 +102,15 @@ def _prep(kc, vc, xq, static_src, static_dest):
     return kc, vc, xq, src, dest, gflag
 
 
+_ROWS_K = _rows_k
+
+
+def native():
+    """The host module for the fused entry points.  Keys and values are described to the kernels by _rows_k in this file's
+    operators; a caller that has put its own function in its place (to see what reaches the kernels) gets these: None."""
+    return _lib.host() if _rows_k is _ROWS_K else None
+
+
 # One grid row per head: the entry points refuse more than 65535 of them (b * h * r, times the chunks per row for the
 # chunked operator).  Heads are independent, so the operators below split such a call along b, then h, run the pieces one
 # after the other and join the results; the pieces keep no forward state (the backward rebuilds it per piece).
@@ -179,6 +189,14 @@ def _gate_grads(b, h, L, src, static_src, static_dest):
 # belongs to.  The note lives on the tensor object and dies with it; a gradient that was accumulated with another one,
 # replaced by a hook or modified in place is another object or version and simply has no (valid) note.
 _NOTE = "_ua_merge_note"
+
+
+def _leave_note(d_mat, d_vec, mat, delta):
+    try:
+        setattr(d_mat, _NOTE, (weakref.ref(d_vec), (mat.data_ptr(), tuple(mat.shape), tuple(mat.stride()), mat._version),
+                               d_mat._version, d_vec._version, delta))
+    except (AttributeError, TypeError):          # a tensor subclass without instance attributes: no note, no shortcut
+        pass
 
 
 def _delta_from_merge(out, g_out, g_denom, L, n):
@@ -359,11 +377,7 @@ def merge_backward(mat, vec, g):
     d_vec = d_vec.to(vec.dtype)
     if delta is None:
         return d_mat, d_vec
-    try:
-        setattr(d_mat, _NOTE, (weakref.ref(d_vec), (mat.data_ptr(), tuple(mat.shape), tuple(mat.stride()), mat._version),
-                               d_mat._version, d_vec._version, delta))
-    except (AttributeError, TypeError):          # a tensor subclass without instance attributes: no note, no shortcut
-        pass
+    _leave_note(d_mat, d_vec, mat, delta)
     return d_mat, d_vec
 
 
@@ -461,12 +475,15 @@ def autotune_affinity(k, src, dest, repeats=5):
 _first_call_tuned = set()
 
 
+def tune_on_first_call():
+    return os.environ.get("UA_AUTOTUNE") == "1"
+
+
 def autotune_on_first_call(kc, vc, xq, static_src, static_dest):
     """UA_AUTOTUNE=1 in the environment: the fused operator tunes itself the first time it meets a table key (dtype,
     padded head dim, r, size buckets of L and b*h), as the reference's @triton.autotune does per key
     (universal_attention_kernel_opt.py:24-44).  Synchronises the device, so not for code under graph capture."""
-    import os
-    if os.environ.get("UA_AUTOTUNE") != "1" or torch.cuda.is_current_stream_capturing():
+    if not tune_on_first_call() or torch.cuda.is_current_stream_capturing():
         return None
     b, h, n, c, d = kc.shape
     L = n * c

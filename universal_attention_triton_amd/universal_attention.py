@@ -18,15 +18,19 @@ from . import universal_attention_autograd as _chunked
 from .universal_attention_autograd import _ChunkedBase
 
 
+def _check_2d(kc, vc, xq, static_src, static_dest):
+    b, h, r, _n, _c, d = xq.shape
+    _, _, n_, c_, _ = kc.shape
+    assert kc.shape == (b, h, n_, c_, d)
+    assert vc.shape == (b, h, n_, c_, d)
+    assert static_src.shape == (b, h, n_, c_)
+    assert static_dest.shape == (b, h, _n, _c)
+
+
 class _CheckedChunked2D(_ChunkedBase):
     @staticmethod
     def forward(kc, vc, xq, static_src, static_dest):
-        b, h, r, _n, _c, d = xq.shape
-        _, _, n_, c_, _ = kc.shape
-        assert kc.shape == (b, h, n_, c_, d)
-        assert vc.shape == (b, h, n_, c_, d)
-        assert static_src.shape == (b, h, n_, c_)
-        assert static_dest.shape == (b, h, _n, _c)
+        _check_2d(kc, vc, xq, static_src, static_dest)
         return _ChunkedBase.forward(kc, vc, xq, static_src, static_dest)
 
     @staticmethod
@@ -43,6 +47,7 @@ class UniversalAttention(_chunked.UniversalAttention):
     """.apply(kc, vc, xq, static_src, static_dest) -> (out, denom), 2-D query layout, with the reference entry point's
     shape checks (Universal_Attention/universal_attention.py:8-13, :35-38)."""
     function = _CheckedChunked2D
+    _check = staticmethod(_check_2d)
 
 
 _fused_bwd = _chunked.kernel_call(lambda *a: ops.fused_backward(*a[:8], state=a[8], prune=a[9], recompute=a[10]), "FusedBackward")
@@ -95,8 +100,11 @@ def universal_attention(kc, vc, xq, static_src, static_dest, return_lse=False, p
     recompute=True (bf16) implies that and also keeps the backward's workspace at O(L*L/16) bytes per head by
     recomputing the score and decay gradients in every kernel instead of exchanging tiles (UA_FLAG_RECOMPUTE)."""
     ops.autotune_on_first_call(kc, vc, xq, static_src, static_dest)          # only with UA_AUTOTUNE=1
-    O, lse, _state = _FusedUniversalAttention.apply(kc, vc, xq, static_src, static_dest, prune, recompute, keep_state)
-    return (O, lse) if return_lse else O
+    host = ops.native()
+    res = host and host.universal(kc, vc, xq, static_src, static_dest, prune, recompute, keep_state)
+    if res is None:      # what the host module does not take: function transforms, odd layouts, many heads, inputs that are errors
+        res = _FusedUniversalAttention.apply(kc, vc, xq, static_src, static_dest, prune, recompute, keep_state)[:2]
+    return res if return_lse else res[0]
 
 
 def attention(q, k, v, causal=True, sm_scale=None, static_src=None, static_dest=None, warp_specialize=True, ac=False):
@@ -108,6 +116,11 @@ def attention(q, k, v, causal=True, sm_scale=None, static_src=None, static_dest=
     B, Hq, L, d = q.shape
     Hkv = k.shape[1]
     assert Hq % Hkv == 0
+    host = ops.native()
+    if host is not None and static_src is not None and not ops.tune_on_first_call():
+        res = host.gen2(q, k, v, static_src, static_dest, not ac)      # reads and writes the heads in their own order
+        if res is not None:
+            return res[0]
     r = Hq // Hkv
     xq = q.view(B, r, Hkv, L, d).transpose(1, 2)                 # [B, H_kv, r, L, d]
     # ac ("activation checkpointing" of the reference: do not keep the bias between forward and backward,

@@ -16,7 +16,7 @@ import contextvars
 import torch
 from torch.autograd import Function
 
-from . import ops
+from . import _lib, ops
 
 
 # Options of the chunked operators.  They are read when a Function is applied (in the caller's thread / context) and
@@ -36,6 +36,7 @@ from . import ops
 #                   and values: every kernel then moves 16 bytes per lane.  True allocates it contiguous like the
 #                   reference does, for callers that `.view()` it; the passes over it are then several times slower.
 _DEFAULTS = {"keep_state": True, "recompute": False, "skip_masked": False, "contiguous_out": False}
+_KEEP = {False: 0, None: 0, "normalisers": 1, True: 2}
 _options = contextvars.ContextVar("ua_chunked_options", default=_DEFAULTS)
 
 
@@ -140,16 +141,34 @@ class UniversalAttention:
 
     @classmethod
     def apply(cls, kc, vc, xq, static_src, static_dest):
-        out, denom, _state = cls.function.apply(kc, vc, xq, static_src, static_dest)
-        return out, denom
+        cls._check(kc, vc, xq, static_src, static_dest)
+        opt = _options.get()
+        res = _lib.host().chunked(kc, vc, xq, static_src, static_dest, _KEEP[opt["keep_state"]], opt["recompute"],
+                                  opt["skip_masked"], opt["contiguous_out"])
+        if res is None:          # what the host module does not take: function transforms, odd layouts, inputs that are errors
+            res = cls.function.apply(kc, vc, xq, static_src, static_dest)[:2]
+        return res
+
+    @staticmethod
+    def _check(kc, vc, xq, static_src, static_dest):
+        b, h, r, l, d = xq.shape
 
 
 class UniversalAttention2(UniversalAttention):
     """2-D layout: xq [b,h,r,_n,_c,d], static_dest [b,h,_n,_c]; the query tiling does not change the result."""
     function = _Chunked2D
 
+    @staticmethod
+    def _check(kc, vc, xq, static_src, static_dest):
+        b, h, r, _n, _c, d = xq.shape
+
 
 class SMVecMatMul(Function):
+    @classmethod
+    def apply(cls, mat, vec):
+        res = _lib.host().merge(mat, vec)
+        return super().apply(mat, vec) if res is None else res
+
     @staticmethod
     def forward(mat, vec):
         return ops.merge_forward(mat, vec)
