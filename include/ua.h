@@ -218,9 +218,8 @@ enum {
                                 two LDS stages, 1 = 8 waves one stage, 2 = 12 waves, 3 = 16 waves, 4 = 4 waves; fp32: one */
   UA_TUNE_CARRY = 16,        /* bias pre-pass of the bf16 operator: 0 = 8 waves x 16 keys per workgroup, 1 = 4 waves,
                                 2 = 4 waves, two key groups of complementary length per workgroup */
-  UA_TUNE_FWD_TILES = 17,    /* bf16 forward over bias tiles: 0 = one 32-query block per wave (256-query workgroups, two
-                                LDS stages), 1 = 16 queries per wave (128-query workgroups, one stage, two per CU),
-                                2 = 16 queries per wave, 64-query workgroups (r = 1 only) */
+  UA_TUNE_FWD_TILES = 17,    /* bf16 forward over bias tiles, one 32-query block per wave: 0 = 4 waves, 1 = 8 waves as four query
+                                slots x two key splits, 2 = two slots x four splits (odd r only) */
   UA_TUNE_BWD_PARTS = 18,    /* key side of the bf16 backward with r > 1: variant i divides the query groups of a kv
                                 head into the i-th smallest divisor of r parts with a sweep each (0 = one shared sweep).
                                 Changes ua_workspace_bytes: set it before sizing the workspace. */

@@ -124,9 +124,16 @@ int heuristic_variant(const ua_desc& d, int slot) {
       const long n4 = Zk * (Lp / 64);      // one to four rounds of the 1024 resident workgroups
       return (n4 >= 1024 && n4 < 4096) ? 2 : 1;
     }
-    case UA_TUNE_FWD_TILES:  // 256-query workgroups need about four per CU to balance; small launches run 64-query pieces
-      if (Zq * (Lp / 256) >= 1024) return 0;
-      return (d.r % 2 == 0 || Zq * (Lp / 128) >= 1536) ? 1 : 2;
+    case UA_TUNE_FWD_TILES: {
+      // 4-wave workgroups (128 / RB queries, two per CU) win once there are three per CU: b = 1 h = 8 r = 4 L = 4096 d = 128 (1024 of
+      // them) 168 us against 194 with two key splits.  With fewer the longest one bounds the launch, and splitting its keys over
+      // the waves is faster: 52 against 46 us at b = 2 h = 16 L = 2048 d = 64 (512), 47 and 39 at b = 1 h = 8 r = 4 L = 1531 (384);
+      // four ways below half a round: 29, 26 and 20 us at b = 1 h = 8 L = 1024 (64).  From 4096 positions on nothing is split: there
+      // a query's result does not depend on how many positions follow it (the splits sum in another order).
+      const long n = Zq * (Lp / 128);
+      if (d.L >= 4096 || n >= 3 * 256) return 0;
+      return d.r % 2 == 1 && n < 128 ? 2 : 1;
+    }
     case UA_TUNE_BWD_PARTS: {
       // Grouped queries: the key-stationary kernel sweeps the r query groups of a kv head in one workgroup, sharing the
       // key-key part of every step (a step of a further group costs about 0.7 of a full one).  Its longest workgroup then
@@ -376,8 +383,9 @@ int pack_inputs(const ua_desc& d, const Layout& l, bool rowmajor, const ua_rows*
   p.lsrc = (float*)(wf + l.lsrc); p.ldest = (float*)(wf + l.ldest);
   p.knorm2 = prune ? (float*)(wf + l.knorm2) : nullptr; p.qnorm2 = prune ? (float*)(wf + l.qnorm2) : nullptr;
   p.Zk = l.Zk; p.d = d.d; p.L = d.L; p.Lp = l.Lp; p.tiled = rowmajor ? 0 : 1;
-  // the chunked kernels work on 32x32 tiles, the fused ones on 16x16 tiles (and read V^T in natural order)
-  p.mode = rowmajor ? TR_PERM16 : TR_PERM32; p.vmode = rowmajor ? TR_PERM16 : TR_NATURAL;
+  // order of the transposed copies: the chunked kernels work on 32x32 tiles, the fused ones on 16x16 tiles; V^T follows the
+  // forward: 32x32 tiles in k_fwd_tiles, natural order for the 16x16 ones
+  p.mode = rowmajor ? TR_PERM16 : TR_PERM32; p.vmode = rowmajor || (l.tiles && l.D <= 128) ? TR_PERM16 : TR_NATURAL;
   UA_HIP(launch_pack_inputs(d.dtype, l.D, p, 2 * l.Zk + l.Zq, s));
   return UA_OK;
 }
@@ -393,7 +401,7 @@ int launch_fwd_for(const ua_desc& d, const Layout& l, char* wf, const ua_rows& O
   UA_HIP(ua::launch_fwd_fused(d.dtype, l.D, variant, wf + l.Qp, wf + l.Kp, wf + l.VT, (const float*)(wf + l.lsrc),
                               (const float*)(wf + l.ldest), (const float*)(wf + l.C), (void*)O.ptr, lse, (float*)(wf + l.lse2),
                               (const int*)(wf + l.reach), d.r, d.L, l.Lp, d.d, l.Zq, rows_out_of(d, O, d.r), s,
-                              l.tiles ? wf + l.Bt : nullptr));
+                              l.tiles ? wf + l.Bt : nullptr, (d.flags & UA_FLAG_PRUNE) != 0));
   return UA_OK;
 }
 int run_fused_fwd_kernels(const ua_desc& d, const Layout& l, char* wf, const ua_rows& O, float* lse, hipStream_t s) {

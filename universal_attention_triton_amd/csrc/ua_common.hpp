@@ -135,6 +135,8 @@ __device__ __forceinline__ void stage_tile(T* __restrict__ lds, const T* __restr
 // w, w+NWAVES, ... and keeps the per-lane source offsets of its instructions in registers.
 // ---------------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
+typedef short v4s16 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) v4s16* lds_v4s16_t;
 
 // A [ROWS][COLS] operand tile in LDS, filled by asynchronous global->LDS loads in units of 16-byte chunks, and
 // read as MFMA operands: lane l takes the 8 k-values of k-group 4q + l/16 of row 16*blk + l%16.
@@ -284,6 +286,31 @@ inline int device_cus() {
 __host__ __device__ __forceinline__ constexpr long tri_bias_row(long tb) { return tb * (tb + 1); }
 __host__ __device__ __forceinline__ constexpr long tri_grad_row(long tq) { return (tq >> 1) * ((tq >> 1) + 1) + ((tq & 1) ? (tq >> 1) + 1 : 0); }
 __host__ __device__ __forceinline__ constexpr long tri_tiles(long nT32) { return nT32 * (nT32 + 1) + 8; }
+// A bias tile (16 keys x 32 queries of fp16, 1 KB) in the order in which the pre-pass holds it: lane (query c, g) of its transposed
+// result tiles owns 16 bytes, keys 4g .. 4g + 3 towards query c and then towards query 16 + c, at unit bias_unit(g, c).  The
+// forward with a query per lane (k_fwd_tiles) fetches 8-byte pieces; the key side of the backward, with a key per lane, reads
+// the tile transposed out of LDS, and the rotation by 4g makes those reads fall on different banks.
+__device__ __forceinline__ constexpr int bias_unit(int g, int c) { return 16 * g + ((c + 4 * g) & 15); }
+// address of the piece that lane `lane` supplies to the transposing read which returns key lane % 16's bias for queries
+// q0 .. q0 + 3 (q0 a multiple of 4 that may differ between the four groups of 16 lanes)
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ const char* bias_piece_at(const char* tile, int q0, int lane) {
+  const int i = lane & 15, kq = i & 3;
+  return tile + (bias_unit(kq, (q0 & 15) + (i >> 2)) << 4) + 8 * (q0 >> 4);
+}
+__device__ __forceinline__ f16x4 bias_piece(const char* tile, int q0, int lane) {
+  return __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s16_t)bias_piece_at(tile, q0, lane)));
+}
+// The same read without the wait: the compiler takes the builtin for one that may touch what the asynchronous copies in
+// flight write and makes it wait for them, which at the start of a step is their whole latency (k_bwd_keys2: 2.93 instead of
+// 2.30 ms).  lds_wait() must stand between the read and the first use, and names the values it completes.
+__device__ __forceinline__ f16x4 bias_piece_nowait(const char* tile, int q0, int lane) {
+  f16x4 r;
+  const unsigned addr = (unsigned)(uintptr_t)(lds_ptr_t)bias_piece_at(tile, q0, lane);
+  asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(r) : "v"(addr));
+  return r;
+}
+__device__ __forceinline__ void lds_wait(f16x4& a, f16x4& b) { asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a), "+v"(b)); }
 // The score / decay gradient tiles of the fused operator are grouped by the workgroup that consumes them (k_bwd_queries3:
 // 8 query tiles = 128 queries): group J = tq / 8 holds, for every 32-key half h = 0 .. 4 J + 3, the eight tiles of its
 // query tiles next to one another, so that the eight waves of the consumer read 8 KB contiguous per tensor and step.
@@ -375,8 +402,6 @@ __device__ __forceinline__ float block_suffix(f32x16& x, int hi) {
 // product contracting over those keys.  bf16 uses ds_read_tr16_b64 (two reads per operand); fp32 has no
 // transposing read and keeps a [16 queries][32 keys] tile written element by element.
 // ---------------------------------------------------------------------------------
-typedef short v4s16 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4s16* lds_v4s16_t;
 template <class T> struct StageT;
 template <> struct StageT<bf16> {
   static constexpr int BYTES = 1024;
@@ -483,12 +508,13 @@ template <bool SUFFIX> __device__ __forceinline__ ScanOps scan_operands(int lane
   }
   return o;
 }
-// y[i] = carry + running sums of the block (values in xb), carry += block total; every register of carry holds the same value
-__device__ __forceinline__ void scan32_mma(const ScanOps& o, const Frag<bf16>& xb, f32x4& carry, f32x4 (&y)[2]) {
+// the same with the roles of the operands exchanged, so that the result tiles are transposed (register v <-> key 4g + v,
+// lane <-> query 16 i + l % 16): y[i] = carry + running sums of the block (values in xb), carry[v] += key 4g + v's block total
+__device__ __forceinline__ void scan32_mma_t(const ScanOps& o, const Frag<bf16>& xb, f32x4& carry, f32x4 (&y)[2]) {
   y[0] = carry; y[1] = carry;
-  mma16(y[0], o.tri[0], xb);
-  mma16(y[1], o.tri[1], xb);
-  mma16(carry, o.ones, xb);
+  mma16(y[0], xb, o.tri[0]);
+  mma16(y[1], xb, o.tri[1]);
+  mma16(carry, xb, o.ones);
 }
 
 // the 4 per-query values of lane group g inside a 16-query tile, from a float array indexed by query

@@ -94,9 +94,7 @@ struct FalseC { static constexpr bool value = false; };
 // is at most max|k| max|q|, and a query's normaliser is at least its own score); a wave stops once all its 16
 // keys are there and records the last 32-query block it reached in reach[z][key tile].
 // BO: instead of the carries C, leave the bias of every visited (16 keys, 32 queries) tile itself, as fp16, in
-// Bt[z][causal triangle of (32-query block, 16-key tile) pairs, see tri_bias_row][1 KB]: lane l of the key tile's wave owns
-// bytes 16 l .. 16 l + 15 = its
-// key's bias towards queries 4g..4g+3 of the block's first 16-query tile, then of the second (g = l / 16).  The
+// Bt[z][causal triangle of (32-query block, 16-key tile) pairs, see tri_bias_row][1 KB], laid out as bias_piece says.  The
 // 16-bit forward and backward kernels then read the bias instead of recomputing the affinity chain; fp16 resolves
 // the bias of every pair that carries weight (|bias| < 16: 2^-7 at worst) to better than the bf16 rounding of the
 // softmax weight itself.
@@ -137,6 +135,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
   ScanOps sc_ops;
   f32x4 carry4 = {0, 0, 0, 0};
   if constexpr (BO) sc_ops = scan_operands<false>(lane);
+  const int bt_lane = bias_unit(g, col) << 4;
   float* Cz = C + (long)z * nT16 * Lp + spos;
   const T* Kz = Kp + (long)z * Lp * D;
   bool dead = false;
@@ -170,10 +169,13 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     constexpr bool MASKED = decltype(masked_c)::value;
     const int tb = first + s;
     if (dead) return;
-    if (__builtin_amdgcn_ballot_w64((BO ? carry4[0] : carry) > thr) == 0) {        // every key of this wave is out of reach from here on
-      dead = true;
-      if (lane == 0) atomicAdd(&n_dead, 1);
-      return;
+    if (knorm2) {          // pruning: is every key of this wave out of reach from here on?
+      const float reaching = BO ? fmaxf(fmaxf(carry4[0], carry4[1]), fmaxf(carry4[2], carry4[3])) : carry;
+      if (__builtin_amdgcn_ballot_w64(reaching > thr) == 0) {
+        dead = true;
+        if (lane == 0) atomicAdd(&n_dead, 1);
+        return;
+      }
     }
     last = tb;
     const T* sK = reinterpret_cast<const T*>(base);
@@ -194,12 +196,12 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     }
     if constexpr (BO) {
       f32x4 y[2];
-      scan32_mma(sc_ops, as_operand16<bf16>(x[0], x[1]), carry4, y);
+      scan32_mma_t(sc_ops, as_operand16<bf16>(x[0], x[1]), carry4, y);
       typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
       f16x8 hb;
 #pragma unroll
       for (int v = 0; v < 4; ++v) { hb[v] = (_Float16)y[0][v]; hb[4 + v] = (_Float16)y[1][v]; }
-      char* dst = reinterpret_cast<char*>(Bt) + (((long)z * tri_tiles(nT) + tri_bias_row(tb) + sb16) << 10) + 16 * lane;
+      char* dst = reinterpret_cast<char*>(Bt) + (((long)z * tri_tiles(nT) + tri_bias_row(tb) + sb16) << 10) + bt_lane;
       __builtin_nontemporal_store(hb, reinterpret_cast<f16x8*>(dst));
     } else {
       float b0, a0, t0, b1, a1, t1;
@@ -496,8 +498,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
           f32x4 sc = {0, 0, 0, 0};
 #pragma unroll
           for (int q = 0; q < NK; ++q) mma16(sc, qf[q], ld8(sK + TN::at(j & 1, col, q, g)));
-          typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-          const f16x4 hb = *reinterpret_cast<const f16x4*>(base + TILES + blk * 4096 + j * 1024 + 16 * lane + 8 * (w & 1));
+          const f16x4 hb = bias_piece(base + TILES + blk * 4096 + j * 1024, 16 * (w & 1) + 4 * g, lane);
           const bool in_reach = reinterpret_cast<const int*>(base + TILES + NW * 2048)[j] >= tbq;
           const bool diag = MASKED && (sbk == tq);
 #pragma unroll
@@ -626,182 +627,174 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
 }
 
 // ---------------------------------------------------------------------------------------------
-// Fused forward of the 16-bit operator with bias tiles, one 32-query block per wave.
-// grid (n or ceil(n / 2), Zk * R / RB) with n = ceil(Lp/32 / NB) workgroup blocks jt (the second form: blocks jt and
-// n - 1 - jt one after the other, see the body), 8 waves, NB = 8 / RB 32-query blocks per workgroup block; wave w owns block NB jt + w / RB of
-// query group w % RB of the workgroup's RB groups (grouped queries share the key and value tiles of a step).
-// Against k_fwd_fused2<BI> (16 queries per wave): every key / value operand read from LDS feeds two matrix
-// instructions (the two 16-query tiles of the block), the staged tiles serve 256 queries instead of 128, and a bias
-// tile of k_carry2<BO> -- (16 keys, 32 queries), lane l owning bytes 16 l .. 16 l + 15 -- is exactly what a lane of
-// this kernel needs for a key tile, so it is loaded straight into registers one step ahead and never touches LDS.
-// 64 keys per step, key tiles visited from the diagonal backwards, two LDS stages.
+// Fused forward of the 16-bit operator over the bias tiles of k_carry2<BO>, head dims up to 128.
+//
+// A wave owns one 32-query block and works on transposed 32x32 score tiles S^T = K Q^T: lane <-> query l % 32, register v <->
+// key 8 (v / 4) + 4 (l / 32) + v % 4.  A query's maximum and sum are then reductions inside a lane plus one exchange with
+// lane ^ 32, the rescaling factor is one value per lane, and a score tile's weights are directly the B operand of
+// O^T = V^T P^T (the packed V^T stores its positions in that order, perm16), so nothing goes through LDS between the
+// two products.
+// NW, KS: the NW waves are NW / KS query slots x KS key splits.  A step covers 32 KT KS keys; wave (slot, ks) takes KT tiles of 32
+// of them, and at the end the KS partial results (max, sum, O) of a slot are combined through LDS.  Launches whose longest
+// workgroup bounds them run with KS = 2 or 4: the same waves sweep a half or a quarter of the steps.
+// RB: query groups of one kv head per workgroup (they share its key and value tiles); NB = NW / KS / RB query blocks.
+// PR: pruning (see k_carry2): key tiles that do not reach a block have no bias tile there, their weights are zero.
+// grid (n or ceil(n / 2), Zk * R / RB) for the n = n_blk workgroup blocks of NB query blocks (the second form: two blocks of
+// complementary length one after the other, the body expanded twice).  Key tiles are visited from the diagonal backwards.
+// Bound by vector issue beside the matrix pipe (10 plain instructions and one transcendental per pair) and the stream of bias tiles:
+// b = 1, h = 32, L = 8192, d = 128 in 0.66 ms, 3.2 GB at 4.8 TB/s; 0.80 ms for the form with a query's weights spread over 16 lanes
+// (two maxima and one sum through lane exchanges per register, weights through LDS).
 // ---------------------------------------------------------------------------------------------
-template <int D, int RB>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_fwd_fused3(RowsOut orow_arg, const bf16* __restrict__ Qp, const bf16* __restrict__ Kp, const bf16* __restrict__ VT, bf16* __restrict__ O,
-             float* __restrict__ lse, float* __restrict__ lse2, const int* __restrict__ reach,
-             int R, int L, int Lp, int d, const _Float16* __restrict__ Bt) {
+template <int D, int RB, int NW, int KS, bool PR>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_fwd_tiles(RowsOut orow_arg, const bf16* __restrict__ Qp, const bf16* __restrict__ Kp, const bf16* __restrict__ VT, bf16* __restrict__ O,
+            float* __restrict__ lse, float* __restrict__ lse2, const int* __restrict__ reach, int R, int L, int Lp, int d,
+            const _Float16* __restrict__ Bt, int n_blk) {
   using T = bf16;
   using TN = Tile<T, 32, D>;
   using TT = Tile<T, D, 32>;
-  using ST = StageT<T>;
   static_assert(RB == 1 || RB == 2 || RB == 4, "1, 2 or 4 query groups per workgroup");
-  constexpr int NK = D / 32, ND = D / 16, NST = 2, NB = 8 / RB;
-  constexpr int TILES = 2 * TN::BYTES + 2 * TT::BYTES, SB = TILES + 1024;     // + reach of the step's four key tiles
+  static_assert((NW == 8 || NW == 4) && (KS == 1 || KS == 2 || KS == 4) && NW / KS >= RB, "4 or 8 waves, 1, 2 or 4 key splits");
+  constexpr int NQ = D / 16, ND = D / 32, NST = 2, QW = NW / KS, NB = QW / RB, KT = KS == 4 ? 1 : 2, TS = KT * KS;
+  constexpr int VOFF = TS * TN::BYTES, SB = 2 * VOFF;        // [TS key tiles][TS value tiles]
   UA_STAGES(SB);
-  __shared__ __attribute__((aligned(256))) char sPbuf[8 * 4 * ST::BYTES];     // per wave: P of (query tile, 32-key half)
-  typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
-  // A workgroup handles two blocks of 32 NB queries one after the other, jt and (number of blocks - 1 - jt): every pair
-  // visits the same number of key tiles, so the launch is a whole number of equal rounds with half the workgroup changes
-  // (see k_bwd_keys2).  The body is expanded once per block.
+  __shared__ float sML[KS > 1 ? NW * 128 : 4];                // (max, sum) of the partial results
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 31, hi = lane >> 5;
   int bx0, zy;
   xcd_map(bx0, zy);
-  const int n_blk = (Lp / 32 + NB - 1) / NB;
   auto sweep = [&](const int jt) __attribute__((always_inline)) {
-  const int zq = RB == 1 ? zy : (zy / (R / RB)) * R + (zy % (R / RB)) * RB + w % RB;
+  const int ks = w / QW, slot = w % QW;
+  const int zq = RB == 1 ? zy : (zy / (R / RB)) * R + (zy % (R / RB)) * RB + slot % RB;
   const int zk = zq / R, nT16 = Lp / 16, nT32 = Lp / 32;
-  const int qb_raw = NB * jt + w / RB;
-  const bool live = qb_raw < nT32;                            // the last workgroup may hold waves past the end
+  const int qb_raw = NB * jt + slot / RB;
+  const bool live = qb_raw < nT32;                            // the last workgroup may hold slots past the end
   const int qb = live ? qb_raw : nT32 - 1;                    // 32-query block of this wave
-  char* sPw = sPbuf + w * 4 * ST::BYTES;
-  Stager<TN, 8> stN;
-  Stager<TT, 8> stT;
+  Stager<TN, NW> stN;
+  Stager<TT, NW> stT;
   stN.init(w, lane, D * (long)sizeof(T), 32);
   stT.init(w, lane, Lp * (long)sizeof(T), D);
-
-  Frag<T> qf[2][NK];
+  Frag<T> qf[NQ];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int q = 0; q < NQ; ++q) qf[q] = ld8(Qp + nat_off<D>(zq, Lp, 32 * qb + col, 16 * q + 8 * hi));
+  f32x16 o[ND];
 #pragma unroll
-    for (int q = 0; q < NK; ++q) qf[i][q] = ld8(Qp + nat_off<D>(zq, Lp, 32 * qb + 16 * i + col, 32 * q + 8 * g));
-  f32x4 o[2][ND], m[2], ls[2];
+  for (int n = 0; n < ND; ++n)
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-#pragma unroll
-    for (int n = 0; n < ND; ++n) o[i][n] = (f32x4){0, 0, 0, 0};
-    m[i] = (f32x4){-1.0e30f, -1.0e30f, -1.0e30f, -1.0e30f};
-    ls[i] = (f32x4){0, 0, 0, 0};
-  }
+    for (int v = 0; v < 16; ++v) o[n][v] = 0.f;
+  float m = -1.0e30f, ls = 0.f;
   const T* Kz = Kp + (long)zk * Lp * D;
   const T* Vz = VT + (long)zk * D * Lp;
-  const int qb_end = min(NB * (jt + 1), nT32);
-  const int n_kt = (qb_end + 1) / 2;                          // key tiles of 64 covering s <= last query of the workgroup
-  // key tiles that cannot reach this workgroup's first query block (see k_carry2) are not visited
-  const int kt_min = first_key_tile(reach + zk * nT16, NB * jt, lane) >> 2;
-  const int n_steps = n_kt - kt_min;
-  // this lane's 16 bytes of key tile 0 of the wave's query block
-  const char* bt_src = reinterpret_cast<const char*>(Bt) + (((long)zk * tri_tiles(nT32) + tri_bias_row(qb)) << 10) + 16 * lane;
-  f16x8 hb_next[4];
-  auto load_bias = [&] __device__ (int kt) __attribute__((always_inline)) {
+  const int* reach_z = reach + zk * nT16;
+  const int n_st = (min(NB * (jt + 1), nT32) + TS - 1) / TS;  // steps that cover the keys up to the workgroup's last query
+  const int st_min = PR ? first_key_tile(reach_z, NB * jt, lane) / (2 * TS) : 0;
+  const int n_steps = n_st - st_min;
+  // this lane's 8-byte pieces (keys 4 hi .. and 8 + 4 hi ..) of key tile 0 of the wave's query block; fetched one step ahead
+  const char* bt_src = reinterpret_cast<const char*>(Bt) + (((long)zk * tri_tiles(nT32) + tri_bias_row(qb)) << 10);
+  const int bt_off0 = 16 * bias_unit(hi, col & 15) + 8 * (col >> 4), bt_off1 = 16 * bias_unit(2 + hi, col & 15) + 8 * (col >> 4);
+  f16x4 hb_next[4 * KT];
+  auto load_bias = [&] __device__ (int st) __attribute__((always_inline)) {
+    const int t0 = st * TS + ks * KT;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      hb_next[j] = __builtin_nontemporal_load(reinterpret_cast<const f16x8*>(bt_src + ((long)(4 * kt + j) << 10)));
+    for (int j = 0; j < KT; ++j) {
+      const char* p = bt_src + ((long)min(t0 + j, qb) << 11);      // tiles after the block's own keys have no bias: any valid one
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        hb_next[4 * j + 2 * h] = __builtin_nontemporal_load(reinterpret_cast<const f16x4*>(p + 1024 * h + bt_off0));
+        hb_next[4 * j + 2 * h + 1] = __builtin_nontemporal_load(reinterpret_cast<const f16x4*>(p + 1024 * h + bt_off1));
+      }
+    }
   };
-
 #define UA_ISSUE(s, base)                                                                   \
   {                                                                                         \
-    const int kt_ = n_kt - 1 - (s);                                                         \
-    stN.issue((base), Kz + (long)(64 * kt_) * D, w);                                        \
-    stN.issue((base) + TN::BYTES, Kz + (long)(64 * kt_ + 32) * D, w);                       \
-    stT.issue((base) + 2 * TN::BYTES, Vz + (long)(2 * kt_) * (32 * D), w);                  \
-    stT.issue((base) + 2 * TN::BYTES + TT::BYTES, Vz + (long)(2 * kt_ + 1) * (32 * D), w);  \
-    if (w == 0) issue_row((base) + TILES, reach + zk * nT16 + 4 * kt_);                      \
+    const long t_ = (long)(n_st - 1 - (s)) * TS;                                            \
+    _Pragma("unroll") for (int i_ = 0; i_ < TS; ++i_) {                                     \
+      stN.issue((base) + i_ * TN::BYTES, Kz + (t_ + i_) * (32 * D), w);                     \
+      stT.issue((base) + VOFF + i_ * TT::BYTES, Vz + (t_ + i_) * (32 * D), w);              \
+    }                                                                                       \
   }
-#define UA_COMPUTE_FAST(s, base) fwd_tile(n_kt - 1 - (s), (base), FalseC())
-#define UA_COMPUTE_SLOW(s, base) fwd_tile(n_kt - 1 - (s), (base), TrueC())
-  auto fwd_tile = [&] __device__ (int kt, const char* base, auto masked_c) {
+#define UA_COMPUTE_FAST(s, base) fwd_step(n_st - 1 - (s), (base), FalseC())
+#define UA_COMPUTE_SLOW(s, base) fwd_step(n_st - 1 - (s), (base), TrueC())
+  auto fwd_step = [&] __device__ (int st, const char* base, auto masked_c) {
     constexpr bool MASKED = decltype(masked_c)::value;
-    // the bias tiles of this step arrived during the previous one; fetch the next step's (a tile row is followed by
-    // the next rows and the tensor by slack, so the loads of the last step stay inside the tensor)
-    f16x8 hb[4];
+    f16x4 hb[4 * KT];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) hb[j] = hb_next[j];
-    if (kt > 0) load_bias(kt - 1);
-    if (MASKED && 4 * kt > 2 * qb + 1) return;         // the whole step lies after this wave's queries
-    const int* rch = reinterpret_cast<const int*>(base + TILES);
-    f32x4 s2[2][4];
+    for (int j = 0; j < 4 * KT; ++j) hb[j] = hb_next[j];
+    if (st > st_min) load_bias(st - 1);
+    const int t0 = st * TS + ks * KT;                         // first of this wave's 32-key tiles
+    if (MASKED && t0 > qb) return;                            // all of them lie after its queries
+    f32x16 x[KT];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int sbk = 4 * kt + j;                      // 16-key tile
-      const T* sK = reinterpret_cast<const T*>(base + (j >> 1) * TN::BYTES);
-      if (!MASKED || sbk <= 2 * qb + 1) {
-        f32x4 sc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+    for (int j = 0; j < KT; ++j) {
+      const T* sK = reinterpret_cast<const T*>(base + (ks * KT + j) * TN::BYTES);
 #pragma unroll
-        for (int q = 0; q < NK; ++q) {
-          const Frag<T> kb = ld8(sK + TN::at(j & 1, col, q, g));
-          mma16(sc[0], qf[0][q], kb);
-          mma16(sc[1], qf[1][q], kb);
+      for (int v = 0; v < 16; ++v) x[j][v] = 0.f;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) mma(x[j], ld8(sK + ((2 * q + hi) * 32 + col) * 8), qf[q]);
+    }
+#pragma unroll
+    for (int j = 0; j < KT; ++j) {
+      const bool diag = MASKED && t0 + j == qb, after = MASKED && t0 + j > qb;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {                           // the tile's two 16-key bias tiles
+        const bool in_reach = !PR || reach_z[min(2 * (t0 + j) + h, nT16 - 1)] >= qb;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int v = 8 * h + e, key = 8 * (v >> 2) + 4 * hi + (v & 3);
+          float y = __builtin_fmaf(x[j][v], kLog2e, (float)hb[4 * j + 2 * h + (e >> 2)][e & 3]);
+          if (PR) y = in_reach ? y : -1.0e30f;
+          if (MASKED) y = (after || (diag && key > col)) ? -1.0e30f : y;
+          x[j][v] = y;
         }
-        const bool in_reach = rch[j] >= qb;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int tq = 2 * qb + i;
-          const bool diag = MASKED && sbk == tq, after = MASKED && sbk > tq;
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const float x = in_reach ? __builtin_fmaf(sc[i][v], kLog2e, (float)hb[j][4 * i + v]) : -1.0e30f;
-            s2[i][j][v] = (MASKED && (after || (diag && 4 * g + v < col))) ? -1.0e30f : x;
-          }
-        }
-      } else {
-        s2[0][j] = (f32x4){-1.0e30f, -1.0e30f, -1.0e30f, -1.0e30f};
-        s2[1][j] = s2[0][j];
       }
     }
-    // online softmax: rescale only when some query of this wave raises its maximum
+    // online softmax; the maximum is raised only where it lags by more than 8 binary orders (weights then stay below 2^8)
+    float mx = x[0][0];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      f32x4 mx;
-      bool grow = false;
+    for (int j = 0; j < KT; ++j)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        mx[v] = allmax16(fmaxf(fmaxf(s2[i][0][v], s2[i][1][v]), fmaxf(s2[i][2][v], s2[i][3][v])));
-        grow |= (mx[v] > m[i][v]);
-      }
-      if (__builtin_amdgcn_ballot_w64(grow) != 0) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const float mn = fmaxf(m[i][v], mx[v]);
-          const float alpha = __builtin_amdgcn_exp2f(m[i][v] - mn);
-          m[i][v] = mn;
-          ls[i][v] *= alpha;
-#pragma unroll
-          for (int n = 0; n < ND; ++n) o[i][n][v] *= alpha;
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        f32x4 p;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          p[v] = __builtin_amdgcn_exp2f(s2[i][j][v] - m[i][v]);
-          ls[i][v] += p[v];
-        }
-        ST::put(sPw + (2 * i + (j >> 1)) * ST::BYTES, 16 * (j & 1) + col, g, p);
-      }
+      for (int v = 0; v < 16; ++v) mx = fmaxf(mx, x[j][v]);
+    {
+      float a, b;
+      swap32(mx, a, b);
+      mx = fmaxf(a, b);
     }
-    // the 32 independent matrix instructions of P V issue back to back while the SIMD's other wave fills the gaps
+    if (__builtin_amdgcn_ballot_w64(mx > m + 8.0f) != 0) {
+      const float mn = mx > m + 8.0f ? mx : m, alpha = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      ls *= alpha;
+#pragma unroll
+      for (int n = 0; n < ND; ++n)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[n][v] *= alpha;
+    }
+    Frag<T> pb[KT][2];
+#pragma unroll
+    for (int j = 0; j < KT; ++j) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        x[j][v] = __builtin_amdgcn_exp2f(x[j][v] - m);
+        ls += x[j][v];
+      }
+      pb[j][0] = as_operand<T>(x[j], 0);
+      pb[j][1] = as_operand<T>(x[j], 1);
+    }
+    // the independent matrix instructions of P V issue back to back while the SIMD's other wave fills the gaps
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int kq = 0; kq < 2; ++kq) {                   // 32 keys per k-step
-      if (!MASKED || 4 * kt + 2 * kq <= 2 * qb + 1) {
-        const T* sV = reinterpret_cast<const T*>(base + 2 * TN::BYTES + kq * TT::BYTES);
-        const Frag<T> pa0 = ST::get(sPw + kq * ST::BYTES, lane), pa1 = ST::get(sPw + (2 + kq) * ST::BYTES, lane);
+    for (int j = 0; j < KT; ++j) {
+      if (MASKED && t0 + j > qb) break;
+      const T* sV = reinterpret_cast<const T*>(base + VOFF + (ks * KT + j) * TT::BYTES);
 #pragma unroll
-        for (int n = 0; n < ND; ++n) {
-          const Frag<T> vb = ld8(sV + TT::at(n, col, 0, g));
-          mma16(o[0][n], pa0, vb);
-          mma16(o[1][n], pa1, vb);
-        }
-      }
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int n = 0; n < ND; ++n) mma(o[n], ld8(sV + ((2 * q + hi) * D + 32 * n + col) * 8), pb[j][q]);
     }
     __builtin_amdgcn_s_setprio(0);
   };
   {
-    // the key tiles visited first hold the diagonal blocks of the waves: those with keys of the workgroup's own blocks
-    const int nslow = min(n_steps, (n_kt - (NB * jt) / 2 + 1) & ~1);
-    if (n_steps > 0) load_bias(n_kt - 1);
+    // the steps visited first hold keys of the workgroup's own blocks
+    const int nslow = min(n_steps, (n_st - (NB * jt) / TS + 1) & ~1);
+    if (n_steps > 0) load_bias(n_st - 1);
     UA_PIPE_START(n_steps, UA_ISSUE);
     UA_PIPE_RANGE(0, nslow, n_steps, UA_ISSUE, UA_COMPUTE_SLOW);
     UA_PIPE_RANGE(nslow, n_steps, n_steps, UA_ISSUE, UA_COMPUTE_FAST);
@@ -809,30 +802,88 @@ k_fwd_fused3(RowsOut orow_arg, const bf16* __restrict__ Qp, const bf16* __restri
 #undef UA_ISSUE
 #undef UA_COMPUTE_FAST
 #undef UA_COMPUTE_SLOW
-  if (!live) return;
-  const RowsOut& orow = late_args<RowsOut>();
-  T* const O_z = O + rows_out(orow, zq);
-  const long o_st = orow.st;
+  __syncthreads();                                            // every wave is done with the stages
+  if constexpr (KS > 1) {
+    // combine the key splits pairwise: the upper half of the splits hands over (every lane its own registers), the lower adds
+    static_assert((NW / 2) * ND * 16 * 256 <= SB, "partial results of half the waves fit a stage");
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int half = KS / 2; half >= 1; half >>= 1) {
+      char* buf = (half == KS / 2 ? stage0 : stage1) + (slot + QW * (ks % half)) * (ND * 16 * 256);
+      float* ml = sML + (slot + QW * (ks % half)) * 128 + (half == KS / 2 ? 0 : NW * 64);
+      if (ks >= half && ks < 2 * half) {
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const float tot = allsum16(ls[i][v]);
-      const float inv = 1.0f / tot;
-      const int t = 32 * qb + 16 * i + 4 * g + v;
-      if (t < L) {
+        for (int n = 0; n < ND; ++n)
 #pragma unroll
-        for (int n = 0; n < ND; ++n) {
-          const int dd = 16 * n + col;
-          if (dd < d) O_z[t * o_st + dd] = cvt<T>(o[i][n][v] * inv);
-        }
+          for (int c = 0; c < 4; ++c)
+            *reinterpret_cast<f32x4*>(buf + ((4 * n + c) * 64 + lane) * 16) = (f32x4){o[n][4 * c], o[n][4 * c + 1], o[n][4 * c + 2], o[n][4 * c + 3]};
+        ml[lane] = m;
+        ml[64 + lane] = ls;
       }
-      if (col == 0) {
-        const float l2v = m[i][v] + __builtin_amdgcn_logf(tot);
-        lse2[(long)zq * Lp + t] = (t < L) ? l2v : 0.f;
-        if (t < L) lse[(long)zq * L + t] = l2v * kLn2;
+      __syncthreads();
+      if (ks < half) {
+        const float m1 = ml[lane], l1 = ml[64 + lane], M = fmaxf(m, m1);
+        const float a0 = __builtin_amdgcn_exp2f(m - M), a1 = __builtin_amdgcn_exp2f(m1 - M);
+        m = M;
+        ls = ls * a0 + l1 * a1;
+#pragma unroll
+        for (int n = 0; n < ND; ++n)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const f32x4 y = *reinterpret_cast<const f32x4*>(buf + ((4 * n + c) * 64 + lane) * 16);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[n][4 * c + e] = o[n][4 * c + e] * a0 + y[e] * a1;
+          }
       }
     }
+    __syncthreads();
+    if (ks != 0) return;
+  }
+  if (!live) return;
+  {
+    float a, b;
+    swap32(ls, a, b);
+    const float tot = a + b, inv = 1.0f / tot;
+    const int t = 32 * qb + col;
+    if (hi == 0) {
+      const float l2v = m + __builtin_amdgcn_logf(tot);
+      lse2[(long)zq * Lp + t] = (t < L) ? l2v : 0.f;
+      if (t < L) lse[(long)zq * L + t] = l2v * kLn2;
+    }
+    // O^T tile -> rows of 2 D bytes in the wave's share of a stage (16-byte pieces exchanged by row, so that neither the 8-byte
+    // writes of a column of queries nor the 16-byte reads of a row meet in one bank) -> pieces of rows
+    constexpr int CH = D / 8;                                 // 16-byte pieces per row
+    static_assert(4 * 32 * D * 2 <= SB, "four waves' rows per stage");
+    char* rows = (slot < 4 ? stage0 : stage1) + (slot & 3) * (32 * D * 2);
+#pragma unroll
+    for (int n = 0; n < ND; ++n)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        union { T h[4]; u32x2 u; } pk;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pk.h[e] = cvt<T>(o[n][4 * c + e] * inv);
+        *reinterpret_cast<u32x2*>(rows + col * (D * 2) + (((4 * n + c) ^ (col & (CH - 1))) << 4) + 8 * hi) = pk.u;
+      }
+    __builtin_amdgcn_wave_barrier();
+    const RowsOut& orow = late_args<RowsOut>();
+    T* const O_z = O + rows_out(orow, zq);
+    const long o_st = orow.st;
+    const bool vec = (d & 7) == 0 && ((reinterpret_cast<uintptr_t>(O) & 15) | ((orow.sb | orow.sh | orow.sr | o_st) & 7)) == 0;
+#pragma unroll
+    for (int i = 0; i < 32 * CH / 64; ++i) {
+      const int row = (i * 64 + lane) / CH, c = (i * 64 + lane) % CH, tt = 32 * qb + row;
+      const u32x4 val = *reinterpret_cast<const u32x4*>(rows + row * (D * 2) + ((c ^ (row & (CH - 1))) << 4));
+      if (tt < L) {
+        if (vec) {
+          if (8 * c < d) *reinterpret_cast<u32x4*>(O_z + tt * o_st + 8 * c) = val;
+        } else {
+          const T* h = reinterpret_cast<const T*>(&val);
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (8 * c + e < d) O_z[tt * o_st + 8 * c + e] = h[e];
+        }
+      }
+    }
+  }
   };
   sweep(n_blk - 1 - bx0);
   if (gridDim.x != n_blk && n_blk - 1 - bx0 != bx0) {     // (launches of few workgroups keep one block each)
@@ -1083,9 +1134,11 @@ __global__ void __launch_bounds__(512) k_bwd_keys2(BwdArgs<T> a) {
     f32x4 (&dB)[2] = MR ? dB_s : dB_l;
     const int tl0 = 32 * tb + 4 * g - spos;        // query position minus key position for (tile 0, v = 0)
     if (!MR || r == 0) {
-      typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-      f16x8 hb;
-      if constexpr (BI) hb = *reinterpret_cast<const f16x8*>(base + TILES + 1024 + w * 1024 + 16 * lane);
+      f16x4 hb[2];
+      if constexpr (BI) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) hb[i] = bias_piece_nowait(base + TILES + 1024 + w * 1024, 16 * i + 4 * g, lane);
+      }
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         f32x4 acc = {0, 0, 0, 0};
@@ -1096,16 +1149,20 @@ __global__ void __launch_bounds__(512) k_bwd_keys2(BwdArgs<T> a) {
         for (int v = 0; v < 4; ++v) {
           gk[i][v] = fmaxf(acc[v], 0.f);
           aff[i][v] = affinity(__builtin_amdgcn_logf(gk[i][v]), lab[v] + la);
-          if constexpr (BI) {
-            bias[i][v] = (float)hb[4 * i + v];
-          } else {
+          if constexpr (!BI) {
             const float l2 = log2_one_minus(aff[i][v]);
             bias[i][v] = (MASKED && diag && tl0 + 16 * i + v <= 0) ? 0.f : l2;
           }
           if (MR) dB[i][v] = 0.f;
         }
       }
-      if constexpr (!BI) {
+      if constexpr (BI) {
+        lds_wait(hb[0], hb[1]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) bias[i][v] = (float)hb[i][v];
+      } else {
         const float cin = stats[128 + 16 * w + col];
         prefix32(bias[0], bias[1], gm);
 #pragma unroll

@@ -47,15 +47,14 @@ hipError_t launch_carry(int dtype, int D, const void* Kp, const float* lsrc, con
                                                                int, int, int, int, ChunkOut<T>, const _Float16*);
 #define UA_INST2(T, D, NST, NW, CH, BI) UA_INST3(T, D, NST, NW, CH, BI, 1)
 #define UA_INST(T, D, NST, NW, CH) UA_INST2(T, D, NST, NW, CH, false)
-UA_INST3(bf16, 64, 1, 8, false, true, 2) UA_INST3(bf16, 128, 1, 8, false, true, 2) UA_INST3(bf16, 64, 1, 8, false, true, 4) UA_INST3(bf16, 128, 1, 8, false, true, 4)
 UA_INST3(bf16, 256, 1, 8, false, true, 2) UA_INST3(bf16, 256, 1, 8, false, true, 4) UA_INST2(bf16, 256, 1, 8, false, true)
-UA_INST2(bf16, 64, 1, 8, false, true) UA_INST2(bf16, 128, 1, 8, false, true) UA_INST2(bf16, 64, 1, 4, false, true) UA_INST2(bf16, 128, 1, 4, false, true)
-template __global__ void k_fwd_fused3<64, 1>(RowsOut, const bf16*, const bf16*, const bf16*, bf16*, float*, float*, const int*, int, int, int, int, const _Float16*);
-template __global__ void k_fwd_fused3<64, 2>(RowsOut, const bf16*, const bf16*, const bf16*, bf16*, float*, float*, const int*, int, int, int, int, const _Float16*);
-template __global__ void k_fwd_fused3<64, 4>(RowsOut, const bf16*, const bf16*, const bf16*, bf16*, float*, float*, const int*, int, int, int, int, const _Float16*);
-template __global__ void k_fwd_fused3<128, 1>(RowsOut, const bf16*, const bf16*, const bf16*, bf16*, float*, float*, const int*, int, int, int, int, const _Float16*);
-template __global__ void k_fwd_fused3<128, 2>(RowsOut, const bf16*, const bf16*, const bf16*, bf16*, float*, float*, const int*, int, int, int, int, const _Float16*);
-template __global__ void k_fwd_fused3<128, 4>(RowsOut, const bf16*, const bf16*, const bf16*, bf16*, float*, float*, const int*, int, int, int, int, const _Float16*);
+#define UA_INSTF_(D, RB, NW, KS, PR)                                                                                              \
+  template __global__ void k_fwd_tiles<D, RB, NW, KS, PR>(RowsOut, const bf16*, const bf16*, const bf16*, bf16*, float*, float*, \
+                                                          const int*, int, int, int, int, const _Float16*, int);
+#define UA_INSTF(RB, NW, KS) UA_INSTF_(64, RB, NW, KS, false) UA_INSTF_(64, RB, NW, KS, true) UA_INSTF_(128, RB, NW, KS, false) UA_INSTF_(128, RB, NW, KS, true)
+UA_INSTF(1, 4, 1) UA_INSTF(2, 4, 1) UA_INSTF(4, 4, 1) UA_INSTF(1, 8, 2) UA_INSTF(2, 8, 2) UA_INSTF(4, 8, 2) UA_INSTF(1, 8, 4)
+#undef UA_INSTF
+#undef UA_INSTF_
 UA_INST(bf16, 64, 1, 8, false) UA_INST(bf16, 64, 2, 8, false) UA_INST(bf16, 64, 2, 12, false) UA_INST(bf16, 64, 2, 16, false)
 UA_INST(bf16, 128, 2, 4, false) UA_INST(bf16, 64, 2, 4, false) UA_INST(bf16, 128, 1, 8, false) UA_INST(bf16, 128, 2, 8, false) UA_INST(bf16, 128, 2, 12, false) UA_INST(bf16, 128, 2, 16, false)
 UA_INST(float, 64, 1, 8, false) UA_INST(float, 128, 1, 8, false)
@@ -73,44 +72,53 @@ static hipError_t fused_t(const void* Qp, const void* Kp, const void* VT, const 
                      (const T*)Kp, (const T*)VT, lsrc, ldest, C, (T*)O, lse, lse2, reach, R, L, Lp, d, ChunkOut<T>{}, none);
   return hipGetLastError();
 }
-// bf16 with bias tiles from launch_carry; variant: UA_TUNE_FWD_TILES
-//   0: k_fwd_fused3, one 32-query block per wave (256-query workgroups, two LDS stages)
-//   1: k_fwd_fused2<BI>, 8-wave workgroups of 128 queries with a single LDS stage, two per CU, which cover each other's waits
-//   2: the same in 64-query pieces (r = 1; small launches are bound by their longest workgroups)
-// grouped queries: the groups of a kv head share the tiles of a 32-query block (see RB)
+// bf16 with bias tiles from launch_carry, head dims up to 128.  prune: the pre-pass left out tiles (UA_FLAG_PRUNE).
+// variant (UA_TUNE_FWD_TILES): 0 = 4 waves, one key split; 1, 2 = 8 waves, two and four.
+template <int D, int RB, int NW, int KS>
+static hipError_t fwd_tiles_t(bool prune, const void* Qp, const void* Kp, const void* VT, void* O, float* lse, float* lse2,
+                              const int* reach, int R, int L, int Lp, int d, int Zq, const RowsOut& orow, hipStream_t s, const void* Bt) {
+  constexpr int nb = NW / KS / RB;
+  const int n_blk = (Lp / 32 + nb - 1) / nb;
+  // Two query blocks per workgroup where these make whole rounds of the CUs, or many: equal workgroups, half as many changes.
+  const long pairs = (long)((n_blk + 1) / 2) * (Zq / RB);
+  // (b = 2 h = 16 L = 2048 d = 64, two key splits: 512 blocks 62 us, 256 pairs 46; one and a half rounds of pairs cost more than
+  // three of single blocks, heaviest first.)
+  const bool pair = pairs >= 4L * device_cus() || (pairs >= device_cus() && pairs % device_cus() == 0);
+  const int gx = pair ? (n_blk + 1) / 2 : n_blk;
+#define UA_FT(PR_)                                                                                                               \
+  hipLaunchKernelGGL((k_fwd_tiles<D, RB, NW, KS, PR_>), dim3(gx, Zq / RB), dim3(64 * NW), 0, s, orow, (const bf16*)Qp, (const bf16*)Kp, \
+                     (const bf16*)VT, (bf16*)O, lse, lse2, reach, R, L, Lp, d, (const _Float16*)Bt, n_blk)
+  if (prune) UA_FT(true); else UA_FT(false);
+#undef UA_FT
+  return hipGetLastError();
+}
+template <int D, int RB>
+static hipError_t fwd_tiles_rb(int variant, bool prune, const void* Qp, const void* Kp, const void* VT, void* O, float* lse, float* lse2,
+                               const int* reach, int R, int L, int Lp, int d, int Zq, const RowsOut& orow, hipStream_t s, const void* Bt) {
+#define UA_ARGS prune, Qp, Kp, VT, O, lse, lse2, reach, R, L, Lp, d, Zq, orow, s, Bt
+  if constexpr (RB == 1) { if (variant == 2) return fwd_tiles_t<D, RB, 8, 4>(UA_ARGS); }
+  return variant == 1 ? fwd_tiles_t<D, RB, 8, 2>(UA_ARGS) : fwd_tiles_t<D, RB, 4, 1>(UA_ARGS);
+#undef UA_ARGS
+}
 template <int D>
-static hipError_t fused_bi(int variant, const void* Qp, const void* Kp, const void* VT, const float* lsrc, const float* ldest,
-                           const float* C, void* O, float* lse, float* lse2, const int* reach, int R, int L,
-                           int Lp, int d, int Zq, const RowsOut& orow, hipStream_t s, const void* Bt) {
-  using T = bf16;
-  if constexpr (D == 256) variant = 1;       // 16 queries per wave: the accumulators of a 32-query block do not fit
-  if constexpr (D != 256) if (variant == 0) {
-    // two query blocks per workgroup once every CU gets at least two of the single ones
-#define UA_F3(RB_)                                                                                                          \
-  do {                                                                                                                      \
-    const int n_blk_ = (Lp / 32 + 8 / RB_ - 1) / (8 / RB_);                                                                 \
-    const int gx_ = (long)n_blk_ * (Zq / RB_) >= 2 * device_cus() ? (n_blk_ + 1) / 2 : n_blk_;                             \
-    hipLaunchKernelGGL((k_fwd_fused3<D, RB_>), dim3(gx_, Zq / RB_), dim3(512), 0, s, orow, (const T*)Qp,                          \
-                       (const T*)Kp, (const T*)VT, (T*)O, lse, lse2, reach, R, L, Lp, d, (const _Float16*)Bt);      \
-  } while (0)
-    if (R % 4 == 0) UA_F3(4);
-    else if (R % 2 == 0) UA_F3(2);
-    else UA_F3(1);
-#undef UA_F3
-    return hipGetLastError();
-  }
-#define UA_SHARED(RB_)                                                                                                     \
-  hipLaunchKernelGGL((k_fwd_fused2<T, D, 1, 8, false, true, RB_>), dim3(Lp / (128 / RB_), Zq / RB_), dim3(512), 0, s, orow, (const T*)Qp, \
-                     (const T*)Kp, (const T*)VT, lsrc, ldest, C, (T*)O, lse, lse2, reach, R, L, Lp, d, ChunkOut<T>{},      \
-                     (const _Float16*)Bt)
+static hipError_t fwd_tiles(int variant, bool prune, const void* Qp, const void* Kp, const void* VT, void* O, float* lse, float* lse2,
+                            const int* reach, int R, int L, int Lp, int d, int Zq, const RowsOut& orow, hipStream_t s, const void* Bt) {
+#define UA_ARGS variant, prune, Qp, Kp, VT, O, lse, lse2, reach, R, L, Lp, d, Zq, orow, s, Bt
+  return R % 4 == 0 ? fwd_tiles_rb<D, 4>(UA_ARGS) : R % 2 == 0 ? fwd_tiles_rb<D, 2>(UA_ARGS) : fwd_tiles_rb<D, 1>(UA_ARGS);
+#undef UA_ARGS
+}
+// head dim above 128: 16 queries per wave (the accumulators of a 32-query block do not fit), 8-wave workgroups of 128 queries; the
+// groups of a kv head share the tiles of a 32-query block (see RB)
+static hipError_t fwd_tiles_256(const void* Qp, const void* Kp, const void* VT, const float* lsrc, const float* ldest, const float* C, void* O,
+                                float* lse, float* lse2, const int* reach, int R, int L, int Lp, int d, int Zq, const RowsOut& orow,
+                                hipStream_t s, const void* Bt) {
+#define UA_SHARED(RB_)                                                                                                           \
+  hipLaunchKernelGGL((k_fwd_fused2<bf16, 256, 1, 8, false, true, RB_>), dim3(Lp / (128 / RB_), Zq / RB_), dim3(512), 0, s, orow,  \
+                     (const bf16*)Qp, (const bf16*)Kp, (const bf16*)VT, lsrc, ldest, C, (bf16*)O, lse, lse2, reach, R, L, Lp, d, \
+                     ChunkOut<bf16>{}, (const _Float16*)Bt)
   if (R % 4 == 0) UA_SHARED(4);
   else if (R % 2 == 0) UA_SHARED(2);
-  else if (variant == 1 || D == 256)
-    hipLaunchKernelGGL((k_fwd_fused2<T, D, 1, 8, false, true>), dim3(Lp / 128, Zq), dim3(512), 0, s, orow, (const T*)Qp, (const T*)Kp,
-                       (const T*)VT, lsrc, ldest, C, (T*)O, lse, lse2, reach, R, L, Lp, d, ChunkOut<T>{}, (const _Float16*)Bt);
-  else if constexpr (D != 256)
-    hipLaunchKernelGGL((k_fwd_fused2<T, D, 1, 4, false, true>), dim3(Lp / 64, Zq), dim3(256), 0, s, orow, (const T*)Qp, (const T*)Kp,
-                       (const T*)VT, lsrc, ldest, C, (T*)O, lse, lse2, reach, R, L, Lp, d, ChunkOut<T>{}, (const _Float16*)Bt);
+  else UA_SHARED(1);
 #undef UA_SHARED
   return hipGetLastError();
 }
@@ -134,10 +142,12 @@ static hipError_t fused_v(int variant, const void* Qp, const void* Kp, const voi
 hipError_t launch_fwd_fused(int dtype, int D, int variant, const void* Qp, const void* Kp, const void* VT,
                             const float* lsrc, const float* ldest, const float* C, void* O, float* lse, float* lse2,
                             const int* reach, int R, int L, int Lp, int d, int Zq, const RowsOut& orow, hipStream_t s,
-                            const void* Bt) {
+                            const void* Bt, bool prune) {
 #define UA_ARGS Qp, Kp, VT, lsrc, ldest, C, O, lse, lse2, reach, R, L, Lp, d, Zq, orow, s
-  if (D == 256) return (dtype == 1 && Bt) ? fused_bi<256>(variant, UA_ARGS, Bt) : hipErrorInvalidValue;
-  if (dtype == 1 && Bt) return D == 64 ? fused_bi<64>(variant, UA_ARGS, Bt) : fused_bi<128>(variant, UA_ARGS, Bt);
+  if (D == 256) return (dtype == 1 && Bt) ? fwd_tiles_256(UA_ARGS, Bt) : hipErrorInvalidValue;
+#define UA_TILES variant, prune, Qp, Kp, VT, O, lse, lse2, reach, R, L, Lp, d, Zq, orow, s, Bt
+  if (dtype == 1 && Bt) return D == 64 ? fwd_tiles<64>(UA_TILES) : fwd_tiles<128>(UA_TILES);
+#undef UA_TILES
   if (dtype == 1) return D == 64 ? fused_v<bf16, 64>(variant, UA_ARGS) : fused_v<bf16, 128>(variant, UA_ARGS);
   return D == 64 ? fused_t<float, 64, 1, 8>(UA_ARGS) : fused_t<float, 128, 1, 8>(UA_ARGS);
 #undef UA_ARGS

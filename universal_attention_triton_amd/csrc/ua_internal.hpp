@@ -38,7 +38,7 @@ int fwd_fused_variants(int dtype, int D);
 hipError_t launch_fwd_fused(int dtype, int D, int variant, const void* Qp, const void* Kp, const void* VT,
                             const float* lsrc, const float* ldest, const float* C, void* O, float* lse, float* lse2,
                             const int* reach, int R, int L, int Lp, int d, int Zq, const RowsOut& orow, hipStream_t s,
-                            const void* Bt = nullptr);   // Bt (bf16): bias tiles of launch_carry; variant is then UA_TUNE_FWD_TILES
+                            const void* Bt = nullptr, bool prune = false);   // Bt (bf16): bias tiles of launch_carry; variant is then UA_TUNE_FWD_TILES, and VT in the order of perm16 for D <= 128
 hipError_t launch_fwd_chunked(int dtype, int D, const void* Qp, const void* Kp, const void* VT, const float* lsrc,
                               const float* ldest, void* out, void* denom, float* lse2, long o_sz, long o_st, long o_sd,
                               long o_si, int R, int L, int Lp, int d, int c, int nch, int Zk, hipStream_t s);

@@ -175,7 +175,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     tr_a = kgrp * 512 + (((4 * hi + (i >> 2)) ^ k4_swz(kgrp)) << 4) + 8 * (i & 1);
     tr_b = tr_a ^ 128;
   }
-  const int bias_lane = TILES + 1024 + w * 2048 + (col >> 4) * 1024 + 16 * (col & 15) + 256 * hi;
+  const int bias_tile = TILES + 1024 + w * 2048 + (col >> 4) * 1024;
 
   // ---- state carried from step to step
   f32x16 F, Gk, dB, run;        // of the block worked on last: dG / dl, relu(G), reverse running sum of dS; sum of dS so far
@@ -272,10 +272,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     Frag<T> bg[2], nbp[2], nbs[2];
     float lb[16];
     load_t16(stats + 64, hi, lb);
-    typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-    // bias: the wave's two fp16 tiles (16 keys x 32 queries each); lane (g, c) of a tile owns 16 bytes: queries 4g..4g+3
-    // of the block's first 16 queries, then of the second
-    const f16x8 hb0 = *reinterpret_cast<const f16x8*>(cur + bias_lane), hb1 = *reinterpret_cast<const f16x8*>(cur + bias_lane + 512);
+    // bias out of the fp16 tile (16 keys x 32 queries) that holds this lane's key: queries 8 j + 4 hi .. + 3
+    f16x4 hb[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) hb[j] = bias_piece(cur + bias_tile, 8 * j + 4 * hi, lane);
     const int tl0 = 32 * tb + 4 * hi - spos;        // query position minus key position for v = 0
     float afv[16];
     __builtin_amdgcn_sched_barrier(0);
@@ -332,7 +332,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
           constexpr int j = v >> 2, m = v & 3;
           if constexpr (ph == 0) { UA_PINV(S, v) UA_PINV(dP, v) }
           if constexpr (ph == 1) {
-            const float bias = (float)((j & 1) ? hb1[4 * (j >> 1) + m] : hb0[4 * (j >> 1) + m]);
+            const float bias = (float)hb[j][m];
             float p = __builtin_amdgcn_exp2f(__builtin_fmaf(S[v], kLog2e, bias));
             if (GEN) p = ((masked && (tl0 + 8 * j + m) < 0) || tb > lane_reach) ? 0.f : p;
             S[v] = p;
