@@ -627,6 +627,217 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
 }
 
 // ---------------------------------------------------------------------------------------------
+// Fused forward in float32: the keys of a query block divided among KS waves.  grid (ceil(Lp / 16 / NS), Zq), NW waves = NS query
+// slots of 16 x KS key splits; a step covers 32 KS keys, wave (slot, ks) takes 32 of them, and at the end the KS partial results
+// (maximum, sum, O) of a slot are combined through LDS.  Key tiles are visited from the diagonal backwards.
+// Bound by the matrix pipe: three products of 16x16x4 instructions (32 cycles each).  A launch lasts as long as its longest workgroup, so
+// the workgroups are small (4 waves, 32 or 16 queries) and the waves of a block share its sweep: with 128 queries per workgroup and
+// no split b = 1, h = 8, L = 2048, d = 64 had 128 workgroups for 256 CUs, two waves of the longest one on each SIMD: 244 us, now 111;
+// h = 4, L = 512, d = 64 (four splits) 63 -> 16.
+// A split whose keys all lie after a query leaves the maximum -1e30 there, and its (finite) sums are weighted by 2^(-1e30 - max) = 0.
+// ---------------------------------------------------------------------------------------------
+template <int D, int NST, int NW, int KS>
+__global__ void __launch_bounds__(64 * NW) k_fwd_split(RowsOut orow_arg, const float* __restrict__ Qp, const float* __restrict__ Kp,
+                                                       const float* __restrict__ VT, const float* __restrict__ lsrc,
+                                                       const float* __restrict__ ldest, const float* __restrict__ C, float* __restrict__ O,
+                                                       float* __restrict__ lse, float* __restrict__ lse2, const int* __restrict__ reach,
+                                                       int R, int L, int Lp, int d) {
+  using T = float;
+  using TN = Tile<T, 32, D>;
+  using TT = Tile<T, D, 32>;
+  using ST = StageT<T>;
+  static_assert((KS == 2 || KS == 4) && NW % KS == 0, "two or four key splits");
+  constexpr int NK = D / 32, ND = D / 16, NS = NW / KS, KEYS = 32 * KS;
+  // [K of the splits][V^T of the splits][per wave: C of its keys: 32f, lsrc: 32f, reach of its (and the neighbour's) key tiles: 4 ints]
+  constexpr int TILES = KS * (TN::BYTES + TT::BYTES), SB = TILES + NW * 1024;
+  UA_STAGES(SB);
+  __shared__ __attribute__((aligned(256))) char sPbuf[NW * ST::BYTES];
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
+  const int slot = w / KS, ks = w % KS;
+  int bx, zq;
+  xcd_map(bx, zq);
+  const int zk = zq / R, nT16 = Lp / 16, jt = (int)gridDim.x - 1 - bx;      // heaviest first
+  const int tq = NS * jt + slot, tbq = tq >> 1;              // Lp is a multiple of 128: every wave has a query block
+  char* sPw = sPbuf + w * ST::BYTES;
+  const GroupMasks gm = group_masks(lane);
+  Stager<TN, NW> stN;
+  Stager<TT, NW> stT;
+  stN.init(w, lane, 0, 32);
+  stT.init(w, lane, 0, D);
+  Frag<T> qf[NK], kf[NK];
+#pragma unroll
+  for (int q = 0; q < NK; ++q) {
+    qf[q] = ld8(Qp + nat_off<D>(zq, Lp, 16 * tq + col, 32 * q + 8 * g));
+    kf[q] = ld8(Kp + nat_off<D>(zk, Lp, 16 * tq + col, 32 * q + 8 * g));
+  }
+  const f32x4 lb = load_t4(ldest + (long)zk * Lp + 16 * tq, g);
+  f32x4 o[ND];
+#pragma unroll
+  for (int n = 0; n < ND; ++n) o[n] = (f32x4){0, 0, 0, 0};
+  f32x4 m = {-1.0e30f, -1.0e30f, -1.0e30f, -1.0e30f}, ls = {0, 0, 0, 0};
+  const T* Kz = Kp + (long)zk * Lp * D;
+  const T* Vz = VT + (long)zk * D * Lp;
+  const int n_kt = (16 * NS * (jt + 1) + KEYS - 1) / KEYS;   // steps' key ranges covering s <= last query of the workgroup
+  const int kt_min = 16 * first_key_tile(reach + zk * nT16, (NS * jt) >> 1, lane) / KEYS;
+  const int n_steps = n_kt - kt_min;
+  const float* row_base;
+  int row_step = KEYS;
+  if (lane < 8) row_base = C + ((long)zk * nT16 + tq) * Lp + 32 * ks + 4 * lane;
+  else if (lane < 16) row_base = lsrc + (long)zk * Lp + 32 * ks + 4 * (lane - 8);
+  else { row_base = reinterpret_cast<const float*>(reach + zk * nT16) + 4 * (ks >> 1); row_step = KEYS / 16; }
+
+#define UA_ISSUE(s, base)                                                                   \
+  {                                                                                         \
+    const int kt_ = n_kt - 1 - (s);                                                         \
+    _Pragma("unroll") for (int h_ = 0; h_ < KS; ++h_) {                                     \
+      stN.issue((base) + h_ * TN::BYTES, Kz + (long)(KEYS * kt_ + 32 * h_) * D, w);         \
+      stT.issue((base) + KS * TN::BYTES + h_ * TT::BYTES, Vz + (long)(KEYS * kt_ + 32 * h_) * D, w); \
+    }                                                                                       \
+    issue_row((base) + TILES + w * 1024, row_base + (long)kt_ * row_step);                  \
+  }
+#define UA_COMPUTE_FAST(s, base) fwd_tile(n_kt - 1 - (s), (base), FalseC())
+#define UA_COMPUTE_SLOW(s, base) fwd_tile(n_kt - 1 - (s), (base), TrueC())
+  auto fwd_tile = [&] __device__ (int kt, const char* base, auto masked_c) {
+    constexpr bool MASKED = decltype(masked_c)::value;
+    const int sb0 = 2 * (KS * kt + ks);                      // first 16-key tile of the wave's half
+    if (MASKED && sb0 > tq) return;                          // every key of the half lies after the wave's queries
+    const float* stats = reinterpret_cast<const float*>(base + TILES + w * 1024);
+    const T* sK = reinterpret_cast<const T*>(base + ks * TN::BYTES);
+    f32x4 s2[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int sbk = sb0 + j;
+      if (!MASKED || sbk <= tq) {
+        const float c = reinterpret_cast<const int*>(stats)[64 + 2 * (ks & 1) + j] >= tbq ? stats[16 * j + col] : -1.0e30f;
+        const float la = stats[32 + 16 * j + col];
+        f32x4 gt = {0, 0, 0, 0}, sc = {0, 0, 0, 0};
+#pragma unroll
+        for (int q = 0; q < NK; ++q) {
+          const Frag<T> kb = ld8(sK + TN::at(j, col, q, g));
+          mma16(gt, kf[q], kb);
+          mma16(sc, qf[q], kb);
+        }
+        const bool diag = MASKED && (sbk == tq);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float l2 = log2_one_minus(affinity(log2_relu(gt[v]), la + lb[v]));
+          gt[v] = (MASKED && diag && 4 * g + v <= col) ? 0.f : l2;
+        }
+        // inclusive prefix over the 16 queries of this wave
+        gt[1] += gt[0]; gt[2] += gt[1]; gt[3] += gt[2];
+        float before, after, tot;
+        group_scan(gt[3], gm, before, after, tot);
+        before += c;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float x = __builtin_fmaf(sc[v], kLog2e, gt[v] + before);
+          s2[j][v] = (MASKED && diag && 4 * g + v < col) ? -1.0e30f : x;
+        }
+      } else {
+        s2[j] = (f32x4){-1.0e30f, -1.0e30f, -1.0e30f, -1.0e30f};
+      }
+    }
+    // online softmax: rescale only when some query of this wave raises its maximum
+    f32x4 mx;
+    bool grow = false;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      mx[v] = allmax16(fmaxf(s2[0][v], s2[1][v]));
+      grow |= (mx[v] > m[v]);
+    }
+    if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float mn = fmaxf(m[v], mx[v]);
+        const float alpha = __builtin_amdgcn_exp2f(m[v] - mn);
+        m[v] = mn;
+        ls[v] *= alpha;
+#pragma unroll
+        for (int n = 0; n < ND; ++n) o[n][v] *= alpha;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      f32x4 p;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        p[v] = __builtin_amdgcn_exp2f(s2[j][v] - m[v]);
+        ls[v] += p[v];
+      }
+      ST::put(sPw, 16 * j + col, g, p);
+    }
+    const T* sV = reinterpret_cast<const T*>(base + KS * TN::BYTES + ks * TT::BYTES);
+    const Frag<T> pa = ST::get(sPw, lane);
+#pragma unroll
+    for (int n = 0; n < ND; ++n) mma16(o[n], pa, ld8(sV + TT::at(n, col, 0, g)));
+  };
+  {
+    // the key ranges visited first hold the diagonal blocks of the waves
+    const int nslow = min(n_steps, (n_kt - (16 * NS * jt) / KEYS + 1) & ~1);
+    UA_PIPE_START(n_steps, UA_ISSUE);
+    UA_PIPE_RANGE(0, nslow, n_steps, UA_ISSUE, UA_COMPUTE_SLOW);
+    UA_PIPE_RANGE(nslow, n_steps, n_steps, UA_ISSUE, UA_COMPUTE_FAST);
+  }
+#undef UA_ISSUE
+#undef UA_COMPUTE_FAST
+#undef UA_COMPUTE_SLOW
+  // combine the splits: [slot][ks - 1][o, maximum, sum: ND + 2 pieces of 64 lanes x 16 bytes] in the first stage
+  static_assert(NS * (KS - 1) * (ND + 2) * 1024 <= SB, "the partial results fit a stage");
+#pragma unroll
+  for (int v = 0; v < 4; ++v) ls[v] = allsum16(ls[v]);
+  __syncthreads();
+  if (ks != 0) {
+    f32x4* p = reinterpret_cast<f32x4*>(stage0) + (slot * (KS - 1) + ks - 1) * (ND + 2) * 64 + lane;
+#pragma unroll
+    for (int n = 0; n < ND; ++n) p[64 * n] = o[n];
+    p[64 * ND] = m;
+    p[64 * (ND + 1)] = ls;
+  }
+  __syncthreads();
+  if (ks != 0) return;
+#pragma unroll
+  for (int i = 0; i < KS - 1; ++i) {
+    const f32x4* p = reinterpret_cast<const f32x4*>(stage0) + (slot * (KS - 1) + i) * (ND + 2) * 64 + lane;
+    const f32x4 m1 = p[64 * ND], l1 = p[64 * (ND + 1)];
+    f32x4 a0, a1;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const float mn = fmaxf(m[v], m1[v]);
+      a0[v] = __builtin_amdgcn_exp2f(m[v] - mn);
+      a1[v] = __builtin_amdgcn_exp2f(m1[v] - mn);
+      m[v] = mn;
+      ls[v] = ls[v] * a0[v] + l1[v] * a1[v];
+    }
+#pragma unroll
+    for (int n = 0; n < ND; ++n) {
+      const f32x4 x = p[64 * n];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) o[n][v] = o[n][v] * a0[v] + x[v] * a1[v];
+    }
+  }
+  const RowsOut& orow = late_args<RowsOut>();
+  T* const O_z = O + rows_out(orow, zq);
+  const long o_st = orow.st;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const float inv = 1.0f / ls[v];
+    const int t = 16 * tq + 4 * g + v;
+    if (t < L) {
+#pragma unroll
+      for (int n = 0; n < ND; ++n) {
+        const int dd = 16 * n + col;
+        if (dd < d) O_z[t * o_st + dd] = o[n][v] * inv;
+      }
+    }
+    if (col == 0) {
+      const float l2v = m[v] + __builtin_amdgcn_logf(ls[v]);
+      lse2[(long)zq * Lp + t] = (t < L) ? l2v : 0.f;
+      if (t < L) lse[(long)zq * L + t] = l2v * kLn2;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 // Fused forward of the 16-bit operator over the bias tiles of k_carry2<BO>, head dims up to 128.
 //
 // A wave owns one 32-query block and works on transposed 32x32 score tiles S^T = K Q^T: lane <-> query l % 32, register v <->
@@ -918,16 +1129,18 @@ __device__ __forceinline__ Frag<T> ld8_tr(const T* tile, int n, int lane) {
 // Key-stationary backward (fused mode).  grid (n or ceil(n / 2), Zk) with n = Lp/128 key groups g (the second form: groups
 // g and n - 1 - g one after the other, see the body); 8 waves; wave w owns keys 128g+16w..+15 and
 // sweeps the 32-query blocks from the last one down to its own; one (query block, query group) per step.
+// NW = 4 (float32): workgroups of 64 keys, see bwd2_mr; h = 8, L = 2048, d = 64 in 291 instead of 465 us.
 // MR = more than one query group per kv head (the decay state of a query block then lives across steps).
 // ---------------------------------------------------------------------------------------------
 // CH: chunked operator (a.c a multiple of 64): the upstream gradient, delta and the normaliser depend on the key's chunk
 // (z index zq*nch + chunk); the 128 keys of a workgroup lie in at most two chunks, whose dO tiles are both staged.
 // TO (16-bit dtypes): leave the score gradient dS and the decay gradient dG of every visited tile, in operand precision,
 // in a.dS_st / a.dG_st for k_bwd_queries3 (which then needs no suffix carries Dsuf).
-template <class T, int D, int NST, bool MR, bool CH, bool TO>
-__global__ void __launch_bounds__(512) k_bwd_keys2(BwdArgs<T> a) {
+template <class T, int D, int NST, bool MR, bool CH, bool TO, int NW = 8>
+__global__ void __launch_bounds__(64 * NW) k_bwd_keys2(BwdArgs<T> a) {
   using TN = Tile<T, 32, D>;
   using TT = Tile<T, D, 32>;
+  static_assert(NW == 8 || (NW == 4 && !CH && !TO), "4 waves: merged operator without tile exchange");
   constexpr int NK = D / 32, ND = D / 16;
   // merged operator with tile exchange: the bias comes from the fp16 tiles of k_carry2<BO> (a.Bt), one 1 KB tile per wave
   // and step after the stats row (the chunked operator keeps the carries C, and Dsuf for the recomputing query side)
@@ -957,13 +1170,13 @@ __global__ void __launch_bounds__(512) k_bwd_keys2(BwdArgs<T> a) {
   // kernel is slower than with a workgroup per key group.
   int bx0, zo;
   xcd_map(bx0, zo);
-  const int n_kg = a.Lp / 128;
+  const int n_kg = a.Lp / (16 * NW);
   auto sweep = [&](const int bx) __attribute__((always_inline)) {
   const int zk = zo / a.key_parts;
   const int Lp = a.Lp, L = a.L, nT16 = Lp / 16, R = MR ? a.R / a.key_parts : 1;
   const long zq0 = (long)zk * a.R + (zo % a.key_parts) * (a.R / a.key_parts);      // first query head of the part
-  const int kg = bx, sb16 = 8 * kg + w, spos = 16 * sb16 + col;      // key group 0 sweeps the most query blocks: first
-  const int nTr = (L + 31) / 32, first = 4 * kg;
+  const int kg = bx, sb16 = NW * kg + w, spos = 16 * sb16 + col;      // key group 0 sweeps the most query blocks: first
+  const int nTr = (L + 31) / 32, first = (NW / 2) * kg;
   if (first >= nTr) return;                      // every key of this workgroup is padding
   // chunked operator: chunk of the workgroup's first key, whether the workgroup reaches into the next one, and which
   // of the two this wave's keys belong to
@@ -977,15 +1190,15 @@ __global__ void __launch_bounds__(512) k_bwd_keys2(BwdArgs<T> a) {
   const bool uniform_part = CH && !a.skip_masked && *a.masked_nz != 0;
   // query blocks beyond the reach of a key tile (see k_carry2) are not visited: the sweep starts at the farthest
   // block any of the 8 waves reaches, and a wave joins in at its own
-  const int* reach_z = a.reach + zk * nT16 + 8 * kg;
+  const int* reach_z = a.reach + zk * nT16 + NW * kg;
   int top = 0;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) top = max(top, reach_z[i]);
+  for (int i = 0; i < NW; ++i) top = max(top, reach_z[i]);
   top = min(top, nTr - 1);
   const int myreach = reach_z[w];
   const GroupMasks gm = group_masks(lane);
-  Stager<TN, 8> stN;
-  Stager<TT, 8> stT;
+  Stager<TN, NW> stN;
+  Stager<TT, NW> stT;
   stN.init(w, lane, D * (long)sizeof(T), 32);
   stT.init(w, lane, Lp * (long)sizeof(T), D);
   // Upstream-gradient tiles.  Normally the packed copy (tiles like those of K and Q).  Chunked operator with a.dO_rows:
@@ -994,11 +1207,11 @@ __global__ void __launch_bounds__(512) k_bwd_keys2(BwdArgs<T> a) {
   // per instruction instead of 1 KB in one piece).
   const bool dO_in_place = CH && TR && a.dO_rows;
   const long dO_len = dO_in_place ? L : Lp;             // rows per (query head, chunk)
-  Stager<TN, 8> stG = stN;
+  Stager<TN, NW> stG = stN;
   if (dO_in_place) {
 #pragma unroll
-    for (int k = 0; k < Stager<TN, 8>::PER; ++k) {
-      const int n = (w + k * 8) * 64 + lane;
+    for (int k = 0; k < Stager<TN, NW>::PER; ++k) {
+      const int n = (w + k * NW) * 64 + lane;
       stG.off[k] = (n & 31) * (D * (int)sizeof(T)) + (n >> 5) * 16;
     }
   }
@@ -1027,7 +1240,7 @@ __global__ void __launch_bounds__(512) k_bwd_keys2(BwdArgs<T> a) {
   const T* Kz = a.Kp + (long)zk * Lp * D;
   const T* KTz = a.KT + (long)zk * D * Lp;
   const float* ldz = a.ldest + (long)zk * Lp;
-  const float* Cz = a.C + (long)zk * nT16 * Lp + 128 * kg;
+  const float* Cz = a.C + (long)zk * nT16 * Lp + 16 * NW * kg;
   float* Dz = a.Dsuf + (long)zk * nT16 * Lp + spos;
   // where this lane's four values of a (16 keys, 16 queries) tile go inside the 1 KB tile of its 32-key half
   static_assert(!TO || sizeof(T) == 2, "tiles are exchanged in 16-bit operand precision");
@@ -1057,7 +1270,7 @@ __global__ void __launch_bounds__(512) k_bwd_keys2(BwdArgs<T> a) {
       else if (lane < 16) src_ = a.delta + zg_ * Lp + 32 * tb_ + 4 * (lane - 8);            \
       else if (lane < 32) src_ = ldz + 32 * tb_ + 4 * (lane & 7);                           \
       else src_ = BI ? ldz + 32 * tb_ + 4 * (lane & 7)   /* no carries with bias tiles */      \
-                     : Cz + (long)(2 * tb_) * Lp + 4 * (lane - 32);                         \
+                     : Cz + (long)(2 * tb_) * Lp + 4 * ((lane - 32) & (4 * NW - 1));        \
       issue_row((base) + TILES, src_);                                                      \
     }                                                                                       \
     if (BI) issue_row_nt((base) + TILES + 1024 + w * 1024, bt_src + (tri_bias_row(tb_) << 10)); \
@@ -1269,8 +1482,8 @@ __global__ void __launch_bounds__(512) k_bwd_keys2(BwdArgs<T> a) {
     }
   };
   {
-    // the last four query blocks of the sweep hold the diagonal blocks of the eight waves
-    const int nblk = top + 1 - first, nfast = ((nblk > 4 ? nblk - 4 : 0) * R) & ~1;
+    // the last NW / 2 query blocks of the sweep hold the diagonal blocks of the waves
+    const int nblk = top + 1 - first, nfast = ((nblk > NW / 2 ? nblk - NW / 2 : 0) * R) & ~1;
     const int total = (uniform_part ? top + 1 : nblk) * R;
     UA_PIPE_START(total, UA_ISSUE);
     UA_PIPE_RANGE(0, nfast, total, UA_ISSUE, UA_COMPUTE_FAST);
@@ -1321,7 +1534,9 @@ __global__ void __launch_bounds__(512) k_bwd_keys2(BwdArgs<T> a) {
 
 // ---------------------------------------------------------------------------------------------
 // Query-stationary backward (fused mode): dQ and the column side of dK, no atomics.
-// grid (Lp/128, Zk); 8 waves; wave w owns queries 16*(8*jt+w)..+15; 64 keys per step.
+// grid (Lp/(16 NS), Zk); NW = NS KS waves: NS slots of 16 queries x KS key splits; 64 keys per step (KS = 2: wave ks of a slot takes
+// half ks of them, and the two waves' sums are added through LDS at the end: float32, bound by the matrix pipe, in 4-wave workgroups of
+// 32 queries at d = 64: h = 8, L = 2048 392 -> 172 us).
 //   dQ[t,:] += sum_s dS[s,t] k_s        dkcol[u,:] += sum_s dg[s,u] k_s
 // dS^T and dg^T pass through a wave-private LDS tile to become A operands.  With r query groups the sweep is
 // repeated per group; dg is linear in dBias, so the groups' contributions to dkcol add up (the cross-tile
@@ -1329,15 +1544,16 @@ __global__ void __launch_bounds__(512) k_bwd_keys2(BwdArgs<T> a) {
 // ---------------------------------------------------------------------------------------------
 // CH: chunked operator (a.c a multiple of 64): the upstream gradient, delta and the normaliser are those of the chunk
 // the step's 64 keys belong to (z index zq*nch + chunk) and are reloaded when the chunk changes.
-template <class T, int D, int NST, bool CH>
-__global__ void __launch_bounds__(512) k_bwd_queries2(BwdArgs<T> a, int d) {
+template <class T, int D, int NST, bool CH, int NW = 8, int KS = 1>
+__global__ void __launch_bounds__(64 * NW) k_bwd_queries2(BwdArgs<T> a, int d) {
   using TN = Tile<T, 32, D>;
   using TT = Tile<T, D, 32>;
-  constexpr int NK = D / 32, ND = D / 16;
+  static_assert(NW % KS == 0 && (KS == 1 || (KS == 2 && !CH)) && (!CH || NW == 8), "key splits: merged operator");
+  constexpr int NK = D / 32, ND = D / 16, NS = NW / KS;
   using ST = StageT<T>;
-  constexpr int TILES = 4 * TN::BYTES + 2 * TT::BYTES, SB = TILES + 8 * 1024;   // + per wave [C: 64f][lsrc: 64f][Dsuf: 64f]
+  constexpr int TILES = 4 * TN::BYTES + 2 * TT::BYTES, SB = TILES + NW * 1024;   // + per wave [C: 64f][lsrc: 64f][Dsuf: 64f]
   UA_STAGES(SB);
-  __shared__ __attribute__((aligned(256))) char sXbuf[8 * 2 * ST::BYTES];
+  __shared__ __attribute__((aligned(256))) char sXbuf[NW * 2 * ST::BYTES];
   // Chunked operator: the stationary upstream rows of the NEXT chunk are copied asynchronously into a wave-private
   // LDS region one step ahead (where the 160 KB of LDS allow it), so that entering a chunk costs an LDS read instead
   // of a round trip to memory; lse2 and delta of the step's chunk travel in the stats row.
@@ -1353,11 +1569,11 @@ __global__ void __launch_bounds__(512) k_bwd_queries2(BwdArgs<T> a, int d) {
   const int Lp = a.Lp, L = a.L, nT16 = Lp / 16, R = a.R;
   const bool split_r = a.split_r != 0;
   const int zk = split_r ? zy / R : zy, r_begin = split_r ? zy % R : 0, r_end = split_r ? r_begin + 1 : R;
-  const int jt = gridDim.x - 1 - bx, tq = 8 * jt + w;
+  const int jt = gridDim.x - 1 - bx, slot = w / KS, ks = w % KS, tq = NS * jt + slot;
   char* sX = sXbuf + w * 2 * ST::BYTES;      // [dS of a 32-key half][dg of that half]
   const GroupMasks gm = group_masks(lane);
-  Stager<TN, 8> stN;
-  Stager<TT, 8> stT;
+  Stager<TN, NW> stN;
+  Stager<TT, NW> stT;
   stN.init(w, lane, D * (long)sizeof(T), 32);
   stT.init(w, lane, Lp * (long)sizeof(T), D);
 
@@ -1373,11 +1589,11 @@ __global__ void __launch_bounds__(512) k_bwd_queries2(BwdArgs<T> a, int d) {
   const T* Kz = a.Kp + (long)zk * Lp * D;
   const T* Vz = a.Vp + (long)zk * Lp * D;
   const T* KTz = a.KT + (long)zk * D * Lp;
-  const int n_kt = 2 * jt + 2;
+  const int n_kt = (16 * NS * (jt + 1) + 63) / 64;
   // key tiles out of reach of this workgroup's first query block are not visited (see k_carry2); inside the range
   // a tile that does not reach this wave's block gets a carry of -1e30, which zeroes its dS and dG
   const int tbq = tq >> 1;
-  const int kt_min = (first_key_tile(a.reach + zk * nT16, 4 * jt, lane) >> 2) & ~1;
+  const int kt_min = (first_key_tile(a.reach + zk * nT16, (NS * jt) >> 1, lane) >> 2) & ~1;
   // per-wave stats row of a step: [C row: 64f][lsrc: 64f][Dsuf row: 64f][reach of the 4 key tiles: 4 ints] and, with
   // the chunked operator, [lse2: 16f][delta: 16f] of this wave's queries in the step's chunk at floats 208 and 224; source of
   // each lane's 16 bytes as base + step * stride (in 4-byte units)
@@ -1398,6 +1614,20 @@ __global__ void __launch_bounds__(512) k_bwd_queries2(BwdArgs<T> a, int d) {
   const int uk0_w = CH ? ((min((16 * tq) / a.c, a.nch - 1) + 1) * a.c) >> 6 : 0;
   const int uk1 = uniform_part ? max(uk0, L >> 6) : uk0;
 
+  // KS == 2: adds what the second wave of a slot has summed to the first one's, through the (free) first stage
+  auto add_split = [&] __device__ (f32x4 (&x)[ND]) __attribute__((always_inline)) {
+    static_assert(KS == 1 || NS * ND * 1024 <= SB, "the partial sums fit a stage");
+    f32x4* p = reinterpret_cast<f32x4*>(stage0) + slot * ND * 64 + lane;
+    if (ks != 0) {
+#pragma unroll
+      for (int n = 0; n < ND; ++n) p[64 * n] = x[n];
+    }
+    __syncthreads();
+    if (ks == 0) {
+#pragma unroll
+      for (int n = 0; n < ND; ++n) x[n] += p[64 * n];
+    }
+  };
   for (int r = r_begin; r < r_end; ++r) {
     const long zq = (long)zk * R + r;
     Frag<T> qt[NK], gt[NK];
@@ -1517,7 +1747,8 @@ __global__ void __launch_bounds__(512) k_bwd_queries2(BwdArgs<T> a, int d) {
       }
       // the 64 keys of the step are handled as two halves of 32 (= one contraction step of the column products);
 #pragma unroll
-      for (int kq = 0; kq < 2; ++kq) {
+      for (int half = 0; half < 2 / KS; ++half) {
+        const int kq = KS == 2 ? ks : half;
         if (MASKED && 4 * kti + 2 * kq > tq) continue;     // wave-uniform: the whole half lies after this wave's queries
 #pragma unroll
         for (int jj = 0; jj < 2; ++jj) {
@@ -1586,8 +1817,8 @@ __global__ void __launch_bounds__(512) k_bwd_queries2(BwdArgs<T> a, int d) {
       }
     };
     {
-      // the last two key tiles hold the diagonal blocks of the eight waves
-      const int nfast = max(n_kt - 2, kt_min), n_all = n_kt + uk1 - uk0;
+      // the last key tiles hold the diagonal blocks of the waves
+      const int nfast = max((16 * NS * jt) / 64, kt_min), n_all = n_kt + uk1 - uk0;
       UA_PIPE_START_AT(kt_min, n_all, UA_ISSUE);
       UA_PIPE_RANGE(kt_min, nfast, n_all, UA_ISSUE, UA_COMPUTE_FAST);
       UA_PIPE_RANGE(nfast, n_all, n_all, UA_ISSUE, UA_COMPUTE_SLOW);
@@ -1596,6 +1827,11 @@ __global__ void __launch_bounds__(512) k_bwd_queries2(BwdArgs<T> a, int d) {
 #undef UA_COMPUTE_FAST
 #undef UA_COMPUTE_SLOW
     __syncthreads();   // the next group's prologue refills stage 0
+    if constexpr (KS == 2) {
+      add_split(dQ);
+      __syncthreads();
+      if (ks != 0) continue;
+    }
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int t = 16 * tq + 4 * g + v;
@@ -1607,6 +1843,10 @@ __global__ void __launch_bounds__(512) k_bwd_queries2(BwdArgs<T> a, int d) {
         }
       }
     }
+  }
+  if constexpr (KS == 2) {
+    add_split(dKc);
+    if (ks != 0) return;
   }
 #pragma unroll
   for (int v = 0; v < 4; ++v) {

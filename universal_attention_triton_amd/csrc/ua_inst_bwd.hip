@@ -24,6 +24,11 @@ static hipError_t bwd_t(const BwdArgsV& v, int Zk, hipStream_t s) {
   template __global__ void k_bwd_keys2<T, D, NST, true, true, false>(BwdArgs<T>);
 UA_INST(bf16, 64, 2) UA_INST(bf16, 128, 2) UA_INST(float, 64, 1) UA_INST(float, 128, 1)
 #undef UA_INST
+#define UA_INST4(D) \
+  template __global__ void k_bwd_keys2<float, D, 1, false, false, false, 4>(BwdArgs<float>); \
+  template __global__ void k_bwd_keys2<float, D, 1, true, false, false, 4>(BwdArgs<float>);
+UA_INST4(64) UA_INST4(128)
+#undef UA_INST4
 template __global__ void k_bwd_keys2<bf16, 64, 2, false, false, true>(BwdArgs<bf16>);
 template __global__ void k_bwd_keys2<bf16, 64, 2, true, false, true>(BwdArgs<bf16>);
 template __global__ void k_bwd_keys2<bf16, 128, 2, false, false, true>(BwdArgs<bf16>);
@@ -37,6 +42,15 @@ template __global__ void k_bwd_keys2<bf16, 128, 2, true, true, true>(BwdArgs<bf1
 
 template <class T, int D, int NST, bool MR, bool CH, bool TO>
 static hipError_t bwd2_mr(const BwdArgs<T>& a, int Lp, int Zk, hipStream_t s, int pair = 0) {
+  // float32 (bound by the matrix pipe, 32 cycles per 16x16x4): workgroups of 4 waves, three per CU at d = 64.  At d = 128 one fills the
+  // LDS of a CU, which pays while the workgroups of 8 waves are fewer than two per CU and their longest bounds the launch (h = 8,
+  // L = 3000: step 3.27 -> 1.92 ms) and costs beyond (h = 16, L = 8192: 18.6 -> 20.8).
+  if constexpr (sizeof(T) == 4 && !CH) {
+    if (D == 64 || (long)(Lp / 128) * Zk < 2L * device_cus()) {
+      hipLaunchKernelGGL((k_bwd_keys2<T, D, NST, MR, CH, TO, 4>), dim3(Lp / 64, Zk), dim3(256), 0, s, a);
+      return hipGetLastError();
+    }
+  }
   // two key groups per workgroup once every CU gets at least two of the single ones
   const int n_kg = Lp / 128, gx = paired_items(n_kg, (long)n_kg * Zk >= 2 * device_cus(), pair);
   hipLaunchKernelGGL((k_bwd_keys2<T, D, NST, MR, CH, TO>), dim3(gx, Zk), dim3(512), 0, s, a);
@@ -82,15 +96,26 @@ hipError_t launch_bwd_keys(int dtype, int D, const BwdArgsV& a, int Zk, int cols
 #define UA_INST(T, D, NST)                                                      \
   template __global__ void k_bwd_queries2<T, D, NST, false>(BwdArgs<T>, int); \
   template __global__ void k_bwd_queries2<T, D, NST, true>(BwdArgs<T>, int);
-UA_INST(bf16, 64, 2) UA_INST(bf16, 128, 2) UA_INST(float, 64, 1) UA_INST(float, 128, 1)
+UA_INST(bf16, 64, 2) UA_INST(bf16, 128, 2)
 #undef UA_INST
+template __global__ void k_bwd_queries2<float, 64, 1, true>(BwdArgs<float>, int);
+template __global__ void k_bwd_queries2<float, 128, 1, true>(BwdArgs<float>, int);
+template __global__ void k_bwd_queries2<float, 64, 1, false, 4, 2>(BwdArgs<float>, int);
+template __global__ void k_bwd_queries2<float, 128, 1, false, 8, 2>(BwdArgs<float>, int);
 
 template <class T, int D, int NST>
 static hipError_t bwdq_t(const BwdArgsV& v, int d, int Zk, hipStream_t s) {
   const BwdArgs<T> a = typed<T>(v);
+  if constexpr (sizeof(T) == 4) {
+    if (!v.chunked) {
+      constexpr int NW = D == 64 ? 4 : 8;
+      hipLaunchKernelGGL((k_bwd_queries2<T, D, NST, false, NW, 2>), dim3(v.Lp / (8 * NW), v.split_r ? Zk * v.R : Zk), dim3(64 * NW), 0, s, a, d);
+      return hipGetLastError();
+    }
+  }
   const dim3 grid(v.Lp / 128, v.split_r ? Zk * v.R : Zk);
   if (v.chunked) hipLaunchKernelGGL((k_bwd_queries2<T, D, NST, true>), grid, dim3(512), 0, s, a, d);
-  else hipLaunchKernelGGL((k_bwd_queries2<T, D, NST, false>), grid, dim3(512), 0, s, a, d);
+  else if constexpr (sizeof(T) == 2) hipLaunchKernelGGL((k_bwd_queries2<T, D, NST, false>), grid, dim3(512), 0, s, a, d);
   return hipGetLastError();
 }
 hipError_t launch_bwd_queries(int dtype, int D, const BwdArgsV& a, int d, int Zk, hipStream_t s) {

@@ -26,6 +26,7 @@ static hipError_t carry_t(const void* Kp, const float* lsrc, const float* ldest,
     hipLaunchKernelGGL((k_carry2<T, D, NST, true, true, 4>), dim3(variant == 2 ? (Lp / 64 + 1) / 2 : Lp / 64, Zk), dim3(256), 0, s, (const T*)Kp, lsrc, ldest, C, Lp, knorm2, qnorm2, R, reach, (_Float16*)Bt);
   else if (tiled && Bt && sizeof(T) == 2) hipLaunchKernelGGL((k_carry2<T, D, NST, true, true>), dim3(Lp / 128, Zk), dim3(512), 0, s, (const T*)Kp, lsrc, ldest, C, Lp, knorm2, qnorm2, R, reach, (_Float16*)Bt);
   else if constexpr (D == 256) return hipErrorInvalidValue;
+  else if (tiled && sizeof(T) == 4) hipLaunchKernelGGL((k_carry2<T, D, NST, true, false, 4>), dim3(Lp / 64, Zk), dim3(256), 0, s, (const T*)Kp, lsrc, ldest, C, Lp, knorm2, qnorm2, R, reach, none);
   else if (tiled) hipLaunchKernelGGL((k_carry2<T, D, NST, true, false>), dim3(Lp / 128, Zk), dim3(512), 0, s, (const T*)Kp, lsrc, ldest, C, Lp, knorm2, qnorm2, R, reach, none);
   else hipLaunchKernelGGL((k_carry2<T, D, NST, false, false>), dim3(Lp / 128, Zk), dim3(512), 0, s, (const T*)Kp, lsrc, ldest, C, Lp, knorm2, qnorm2, R, reach, none);
   return hipGetLastError();
@@ -57,8 +58,12 @@ UA_INSTF(1, 4, 1) UA_INSTF(2, 4, 1) UA_INSTF(4, 4, 1) UA_INSTF(1, 8, 2) UA_INSTF
 #undef UA_INSTF_
 UA_INST(bf16, 64, 1, 8, false) UA_INST(bf16, 64, 2, 8, false) UA_INST(bf16, 64, 2, 12, false) UA_INST(bf16, 64, 2, 16, false)
 UA_INST(bf16, 128, 2, 4, false) UA_INST(bf16, 64, 2, 4, false) UA_INST(bf16, 128, 1, 8, false) UA_INST(bf16, 128, 2, 8, false) UA_INST(bf16, 128, 2, 12, false) UA_INST(bf16, 128, 2, 16, false)
-UA_INST(float, 64, 1, 8, false) UA_INST(float, 128, 1, 8, false)
 UA_INST(bf16, 64, 2, 8, true) UA_INST(bf16, 128, 2, 8, true) UA_INST(float, 64, 1, 8, true) UA_INST(float, 128, 1, 8, true)
+#define UA_INSTS(D, NST, NW, KS)                                                                                                      \
+  template __global__ void k_fwd_split<D, NST, NW, KS>(RowsOut, const float*, const float*, const float*, const float*, const float*, \
+                                                       const float*, float*, float*, float*, const int*, int, int, int, int);
+UA_INSTS(64, 1, 4, 2) UA_INSTS(128, 1, 4, 2) UA_INSTS(64, 2, 4, 4) UA_INSTS(128, 1, 4, 4)
+#undef UA_INSTS
 #undef UA_INST
 #undef UA_INST2
 #undef UA_INST3
@@ -122,8 +127,20 @@ static hipError_t fwd_tiles_256(const void* Qp, const void* Kp, const void* VT, 
 #undef UA_SHARED
   return hipGetLastError();
 }
+// float32: two key splits, or four where those workgroups (of 32 queries) would leave CUs without one
+template <int D>
+static hipError_t fwd_split(const void* Qp, const void* Kp, const void* VT, const float* lsrc, const float* ldest, const float* C, void* O,
+                            float* lse, float* lse2, const int* reach, int R, int L, int Lp, int d, int Zq, const RowsOut& orow, hipStream_t s) {
+#define UA_FS(NST_, KS_)                                                                                                       \
+  hipLaunchKernelGGL((k_fwd_split<D, NST_, 4, KS_>), dim3(Lp / (64 / KS_), Zq), dim3(256), 0, s, orow, (const float*)Qp, (const float*)Kp, \
+                     (const float*)VT, lsrc, ldest, C, (float*)O, lse, lse2, reach, R, L, Lp, d)
+  if ((long)(Lp / 32) * Zq < device_cus()) UA_FS((D == 64 ? 2 : 1), 4);
+  else UA_FS(1, 2);
+#undef UA_FS
+  return hipGetLastError();
+}
 // variants (bf16): 0 = 8 waves, double-buffered stages; 1 = 8 waves, single stage; 2 = 12 waves; 3 = 16 waves
-// (both double-buffered).  fp32 always runs 8 waves with a single stage.
+// (both double-buffered).
 int fwd_fused_variants(int dtype, int D) { (void)D; return dtype == 1 ? 5 : 1; }
 template <class T, int D>
 static hipError_t fused_v(int variant, const void* Qp, const void* Kp, const void* VT, const float* lsrc, const float* ldest,
@@ -149,7 +166,7 @@ hipError_t launch_fwd_fused(int dtype, int D, int variant, const void* Qp, const
   if (dtype == 1 && Bt) return D == 64 ? fwd_tiles<64>(UA_TILES) : fwd_tiles<128>(UA_TILES);
 #undef UA_TILES
   if (dtype == 1) return D == 64 ? fused_v<bf16, 64>(variant, UA_ARGS) : fused_v<bf16, 128>(variant, UA_ARGS);
-  return D == 64 ? fused_t<float, 64, 1, 8>(UA_ARGS) : fused_t<float, 128, 1, 8>(UA_ARGS);
+  return D == 64 ? fwd_split<64>(UA_ARGS) : fwd_split<128>(UA_ARGS);
 #undef UA_ARGS
 }
 
