@@ -17,20 +17,33 @@
 
 namespace ua {
 
+// Waves per workgroup of the 16-bit-capable kernels, 16 positions each.  Their steps are bound by latency (a step of the backward's key
+// kernel has 1000 cycles of work per wave and lasts 4000): two or three workgroups of 4 waves on a CU fill each other's gaps
+// where one of 8 waves waits as a whole.  h = 8, L = 4096, d = 128: forward 138 -> 115 us, key side 254 -> 230 and, with the stores of a
+// step left in flight over the next barrier, 186; column side 80 -> 70.
+constexpr int kAffWaves = 4;
+// Head and key group of a workgroup.  Every XCD gets whole heads (xcd_map).  A launch with one workgroup per key group runs the first
+// half of a head's groups from the longest sweep on and the second half from the shortest, so that the groups that share a
+// CU add up to the same length.
+__device__ __forceinline__ void aff_group(int n, int& bx, int& z) {
+  xcd_map(bx, z);
+  if ((int)gridDim.x == n && 2 * bx >= n) bx = n - 1 - (bx - n / 2);
+}
+
 // The pipeline macros of ua_fused.hpp are private to that header; these kernels use a two-stage loop of their own,
 // unrolled by two over two distinct LDS objects, and take one key group per workgroup or two of complementary length.
-// grid (Lp/128 or half of it, Z), 8 waves; wave w owns keys 16*(8*bx+w)..+15 and sweeps the 32-query blocks from its own on.
-// The (32 queries, 128 keys) block of a step goes through LDS so that it leaves as whole rows of 256 (bf16) or 512
+// grid (Lp/NKEY or half of it, Z), NW waves; wave w owns keys 16*(NW*bx+w)..+15 and sweeps the 32-query blocks from its own on.
+// The (32 queries, NKEY keys) block of a step goes through LDS so that it leaves as whole rows of 128 (bf16) or 256
 // bytes, 16 bytes per lane (vec: rows of aff start 16-byte aligned); the block of step s is written out during step
 // s + 1.  The rows above the workgroup's first block (queries before all of its keys) are filled the same way.
 template <class T, int D>
-__global__ void __launch_bounds__(512) k_aff_fwd(const T* __restrict__ Kp, const float* __restrict__ lsrc,
+__global__ void __launch_bounds__(64 * kAffWaves) k_aff_fwd(const T* __restrict__ Kp, const float* __restrict__ lsrc,
                                                  const float* __restrict__ ldest, T* __restrict__ aff, int L, int Lp, int vec) {
   using TN = Tile<T, 32, D>;
-  constexpr int NK = D / 32, SB = TN::BYTES + 1024;
+  constexpr int NW = kAffWaves, NKEY = 16 * NW, NK = D / 32, SB = TN::BYTES + 1024;
   constexpr int EPV = 16 / (int)sizeof(T);            // elements per 16-byte vector
-  constexpr int ROWB = 128 * (int)sizeof(T) + 16;     // bytes per row of the block in LDS (padded: no bank conflicts)
-  constexpr int TPR = 128 / EPV, RPP = 512 / TPR;     // threads per row, rows per pass of the workgroup
+  constexpr int ROWB = NKEY * (int)sizeof(T) + 16;     // bytes per row of the block in LDS (padded: no bank conflicts)
+  constexpr int TPR = NKEY / EPV, RPP = 64 * NW / TPR;     // threads per row, rows per pass of the workgroup
   // distinct objects per stage: the compiler then knows that the asynchronous loads filling one stage do not alias
   // the reads of the other and does not wait for them
   __shared__ __attribute__((aligned(1024))) char stage0[SB];
@@ -38,12 +51,14 @@ __global__ void __launch_bounds__(512) k_aff_fwd(const T* __restrict__ Kp, const
   __shared__ __attribute__((aligned(16))) char oblk0[32 * ROWB];
   __shared__ __attribute__((aligned(16))) char oblk1[32 * ROWB];
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
-  const int bx0 = blockIdx.x, z = blockIdx.y, n_kg = Lp / 128;
+  const int n_kg = Lp / NKEY;
+  int bx0, z;
+  aff_group(n_kg, bx0, z);
   const GroupMasks gm = group_masks(lane);
   auto sweep = [&](const int bx) __attribute__((always_inline)) {
-  const int nT = Lp / 32, sb16 = 8 * bx + w, first = 4 * bx, own = sb16 >> 1;
+  const int nT = Lp / 32, sb16 = NW * bx + w, first = (NW / 2) * bx, own = sb16 >> 1;
   const int spos = 16 * sb16 + col;
-  Stager<TN, 8> st;
+  Stager<TN, NW> st;
   st.init(w, lane, D * (long)sizeof(T), 32);
   Frag<T> ks[NK];
 #pragma unroll
@@ -52,8 +67,8 @@ __global__ void __launch_bounds__(512) k_aff_fwd(const T* __restrict__ Kp, const
   const T* Kz = Kp + (long)z * Lp * D;
   T* az = aff + (long)z * L * L;
   const T fill = cvt<T>(kNegFill);
-  // this thread's piece of a row of the workgroup's 128 columns
-  const int prow = tid / TPR, s0 = 128 * bx + EPV * (tid % TPR);
+  // this thread's piece of a row of the workgroup's columns
+  const int prow = tid / TPR, s0 = NKEY * bx + EPV * (tid % TPR);
   // stores this thread's 16 bytes of row t (handed over in registers: a pointer to them would send them through scratch
   // memory, and every store would wait for the one before it)
   auto put_piece = [&] __device__ (int t, const uint4 val) __attribute__((always_inline)) {
@@ -90,6 +105,7 @@ __global__ void __launch_bounds__(512) k_aff_fwd(const T* __restrict__ Kp, const
       put_piece(32 * tb + r0 + prow, *reinterpret_cast<const uint4*>(blk + (r0 + prow) * ROWB + 16 * (tid % TPR)));
   };
   float carry = 0.f;
+  bool stored = false;
   const int total = nT - first;
   auto issue = [&] __device__ (int s, char* base) __attribute__((always_inline)) {
     st.issue(base, Kz + (long)32 * (first + s) * D, w);
@@ -97,10 +113,13 @@ __global__ void __launch_bounds__(512) k_aff_fwd(const T* __restrict__ Kp, const
   };
   issue(0, stage0);
   auto step = [&] __device__ (const int s, char* cur, char* nxt, char* ob_cur, char* ob_prev) __attribute__((always_inline)) {
-    wait_async_loads();
+    // the stores of a block that lies inside the matrix stay in flight over the next barrier (32 / RPP of them per wave)
+    wait_loads_before_stores<32 / RPP>(stored);
     __syncthreads();
-    if (s > 0) flush(first + s - 1, ob_prev);
     if (s + 1 < total) issue(s + 1, nxt);
+    stores_after_loads();
+    if (s > 0) flush(first + s - 1, ob_prev);
+    stored = s > 0 && vec && 32 * (first + s) <= L && NKEY * (bx + 1) <= L;
     const int tb = first + s;
     if (32 * tb >= L) return;                        // padding rows only: nothing to write
     char* mine = ob_cur + (16 * w + col) * (int)sizeof(T);
@@ -262,34 +281,36 @@ __global__ void __launch_bounds__(512) k_aff_bwd_side(const T* __restrict__ Kp, 
 // ---------------------------------------------------------------------------------------------
 // 16-bit dtypes, rows of daff 16-byte aligned: the backward without the L x L float32 tensor DL.
 // k_aff_bwd_keys is key-stationary like k_aff_bwd_side<false> but sweeps the query blocks from the last one down to
-// its own, carrying the reverse running sum per key (dcar), and reads the (32 queries, 128 keys) block of daff of a step
-// through LDS (rows of 256 bytes, 16 bytes per lane).  It leaves W = dl F as bf16 tiles of 1 KB — (32 keys, 16
+// its own, carrying the reverse running sum per key (dcar), and reads the (32 queries, NKEY keys) block of daff of a step
+// through LDS (rows of 128 bytes, 16 bytes per lane).  It leaves W = dl F as bf16 tiles of 1 KB — (32 keys, 16
 // queries) in the LDS image of StageT, row after row of the causal triangle (tri_grad_row) — and k_aff_bwd_cols, one
 // wave per 16 positions u, turns its row of tiles into the column side sum_s W[s,u] k_s with nothing but matrix products.
-//   grid (Lp/128, Z), 8 waves each.
+//   grid (Lp/NKEY or half of it, Z), NW waves each.
 // ---------------------------------------------------------------------------------------------
 template <class T, int D>
-__global__ void __launch_bounds__(512) k_aff_bwd_keys(const T* __restrict__ Kp, const T* __restrict__ KT,
+__global__ void __launch_bounds__(64 * kAffWaves) k_aff_bwd_keys(const T* __restrict__ Kp, const T* __restrict__ KT,
                                                       const float* __restrict__ lsrc, const float* __restrict__ ldest,
                                                       const T* __restrict__ daff, T* __restrict__ Wst, float* __restrict__ row,
                                                       float* __restrict__ gsum, int L, int Lp) {
   static_assert(sizeof(T) == 2, "tiles are exchanged in 16-bit operand precision");
   using TN = Tile<T, 32, D>;
   using TT = Tile<T, D, 32>;
-  constexpr int NK = D / 32, ND = D / 16, DB = 32 * 128 * (int)sizeof(T), SB = TN::BYTES + TT::BYTES + DB + 1024;
+  constexpr int NW = kAffWaves, NKEY = 16 * NW, PPR = NKEY / 8, NK = D / 32, ND = D / 16, DB = 32 * NKEY * (int)sizeof(T), SB = TN::BYTES + TT::BYTES + DB + 1024;
   // distinct objects per stage (see k_aff_fwd)
   __shared__ __attribute__((aligned(1024))) char stage0[SB];
   __shared__ __attribute__((aligned(1024))) char stage1[SB];
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
-  const int bx0 = blockIdx.x, z = blockIdx.y, n_kg = Lp / 128;
+  const int n_kg = Lp / NKEY;
+  int bx0, z;
+  aff_group(n_kg, bx0, z);
   const int nTr = (L + 31) / 32;
   const GroupMasks gm = group_masks(lane);
   auto sweep = [&](const int bx) __attribute__((always_inline)) {
-    const int first = 4 * bx;
+    const int first = (NW / 2) * bx;
     if (first >= nTr) return;                      // every key of this group is padding
-    const int sb16 = 8 * bx + w, own = sb16 >> 1, spos = 16 * sb16 + col;
-    Stager<TN, 8> stN;
-    Stager<TT, 8> stT;
+    const int sb16 = NW * bx + w, own = sb16 >> 1, spos = 16 * sb16 + col;
+    Stager<TN, NW> stN;
+    Stager<TT, NW> stT;
     stN.init(w, lane, D * (long)sizeof(T), 32);
     stT.init(w, lane, Lp * (long)sizeof(T), D);
     Frag<T> ki[NK];
@@ -303,11 +324,12 @@ __global__ void __launch_bounds__(512) k_aff_bwd_keys(const T* __restrict__ Kp, 
 #pragma unroll
     for (int n = 0; n < ND; ++n) acc_o[n] = (f32x4){0, 0, 0, 0};
     float gs = 0.f, dcar = 0.f;
+    bool stored = false;                           // the step's two stores have been issued after the next step's loads
     // where this lane's four values of a (16 keys, 16 queries) tile go inside the 1 KB tile of its 32-key half
     char* wz = reinterpret_cast<char*>(Wst) + (long)z * (tri_tiles(Lp >> 5) << 10) + ((long)(sb16 >> 1) << 10) +
                StageT<bf16>::addr(perm32(16 * (sb16 & 1) + col), 8 * g);
-    // this lane's 16 bytes of the daff block of a step: row 4 w + g, keys 128 bx + 8 col ..
-    const int drow = 4 * w + g, dcol = 128 * bx + 8 * col;
+    // this lane's 16 bytes of the daff block of a step
+    const int drow = (64 * w + lane) / PPR, dcol = NKEY * bx + 8 * (lane % PPR);
     const int total = nTr - first;
     auto issue = [&] __device__ (int s, char* base) __attribute__((always_inline)) {
       const int tb = nTr - 1 - s;
@@ -319,7 +341,8 @@ __global__ void __launch_bounds__(512) k_aff_bwd_keys(const T* __restrict__ Kp, 
     };
     issue(0, stage0);
     auto step = [&] __device__ (const int s, const char* base, char* nxt) __attribute__((always_inline)) {
-      wait_async_loads();
+      wait_loads_before_stores<2>(stored);
+      stored = false;
       __syncthreads();
       if (s + 1 < total) issue(s + 1, nxt);
       const int tb = nTr - 1 - s;
@@ -342,7 +365,7 @@ __global__ void __launch_bounds__(512) k_aff_bwd_keys(const T* __restrict__ Kp, 
           aff[i2][v] = affinity(__builtin_amdgcn_logf(gk[i2][v]), li + lj[v]);
           // aff[t][s] depends on the inputs only for t > s (it is a constant elsewhere)
           const bool valid = t > spos && t < L && spos < L;
-          W[i2][v] = valid ? __uint_as_float((unsigned)sD[r * 128] << 16) : 0.f;
+          W[i2][v] = valid ? __uint_as_float((unsigned)sD[r * NKEY] << 16) : 0.f;
         }
       }
       float t1;
@@ -359,9 +382,11 @@ __global__ void __launch_bounds__(512) k_aff_bwd_keys(const T* __restrict__ Kp, 
       dcar += tot;
       const Frag<T> b = as_operand16<T>(W[0], W[1]);
       {   // query tiles 2 tb and 2 tb + 1: their rows of tiles start tb + 1 tiles apart
+        stores_after_loads();
         char* p = wz + (tri_grad_row(2 * tb) << 10);
         __builtin_nontemporal_store(reinterpret_cast<const u32x2*>(&b)[0], reinterpret_cast<u32x2*>(p));
         __builtin_nontemporal_store(reinterpret_cast<const u32x2*>(&b)[1], reinterpret_cast<u32x2*>(p + ((long)(tb + 1) << 10)));
+        stored = true;
       }
 #pragma unroll
       for (int n = 0; n < ND; ++n) mma16(acc_o[n], ld8(sKT + TT::at(n, col, 0, g)), b);
@@ -391,31 +416,33 @@ __global__ void __launch_bounds__(512) k_aff_bwd_keys(const T* __restrict__ Kp, 
   }
 }
 
-// colp[z][u][:] = sum_{s<u} W[s,u] k_s from the tiles of k_aff_bwd_keys; wave w owns positions 16*(8*jt+w)..+15 and
+// colp[z][u][:] = sum_{s<u} W[s,u] k_s from the tiles of k_aff_bwd_keys; wave w owns positions 16*(NW*jt+w)..+15 and
 // streams its own row of tiles (two 32-key halves per step of 64 keys) straight into LDS.
 template <class T, int D>
-__global__ void __launch_bounds__(512) k_aff_bwd_cols(const T* __restrict__ KT, const T* __restrict__ Wst, float* __restrict__ colp,
+__global__ void __launch_bounds__(64 * kAffWaves) k_aff_bwd_cols(const T* __restrict__ KT, const T* __restrict__ Wst, float* __restrict__ colp,
                                                       int L, int Lp) {
   static_assert(sizeof(T) == 2, "tiles are exchanged in 16-bit operand precision");
   using TT = Tile<T, D, 32>;
   using ST = StageT<T>;
-  constexpr int ND = D / 16, TILES = 2 * TT::BYTES, WAVE = 2 * ST::BYTES, SB = TILES + 8 * WAVE;
+  constexpr int NW = kAffWaves, ND = D / 16, TILES = 2 * TT::BYTES, WAVE = 2 * ST::BYTES, SB = TILES + NW * WAVE;
   // distinct objects per stage (see k_aff_fwd)
   __shared__ __attribute__((aligned(1024))) char stage0[SB];
   __shared__ __attribute__((aligned(1024))) char stage1[SB];
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
-  const int z = blockIdx.y, n_blk = Lp / 128, bx0 = blockIdx.x;
+  const int n_blk = Lp / (16 * NW);
+  int bx0, z;
+  aff_group(n_blk, bx0, z);
   auto sweep = [&](const int jt) __attribute__((always_inline)) {
-    const int tq = 8 * jt + w;
-    if (128 * jt >= L) return;                     // padding positions only
-    Stager<TT, 8> stT;
+    const int tq = NW * jt + w;
+    if (16 * NW * jt >= L) return;                     // padding positions only
+    Stager<TT, NW> stT;
     stT.init(w, lane, Lp * (long)sizeof(T), D);
     f32x4 dKc[ND];
 #pragma unroll
     for (int n = 0; n < ND; ++n) dKc[n] = (f32x4){0, 0, 0, 0};
     const T* KTz = KT + (long)z * D * Lp;
     const char* pW = reinterpret_cast<const char*>(Wst) + (long)z * (tri_tiles(Lp >> 5) << 10) + (tri_grad_row(tq) << 10) + 16 * lane;
-    const int n_kt = 2 * jt + 2;
+    const int n_kt = (16 * NW * (jt + 1) + 63) / 64;
     auto issue = [&] __device__ (int s, char* base) __attribute__((always_inline)) {
       stT.issue(base, KTz + (long)(64 * s) * D, w);
       stT.issue(base + TT::BYTES, KTz + (long)(64 * s + 32) * D, w);

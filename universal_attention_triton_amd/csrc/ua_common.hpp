@@ -319,6 +319,14 @@ __host__ __device__ __forceinline__ constexpr long grp_tile(long tq, long h) { r
 __host__ __device__ __forceinline__ constexpr long grp_tiles(long nT32) { return 16 * (nT32 >> 2) * ((nT32 >> 2) + 1) + 8; }
 
 __device__ __forceinline__ void wait_async_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// The same where the wave has issued (at least) N stores after the loads it waits for: vector memory operations are counted down in
+// order, so the stores may stay in flight.  Waiting for them puts their round trip into every step.  stores_after_loads() stands
+// between the loads and the stores and keeps the compiler from exchanging them.
+template <int N> __device__ __forceinline__ void wait_loads_before_stores(bool stored) {
+  if (stored) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+  else wait_async_loads();
+}
+__device__ __forceinline__ void stores_after_loads() { asm volatile("" ::: "memory"); }
 
 // Column order of the transposed ([feature][position]) working tensors: inside every group of 16
 // positions bits 2 and 3 are swapped, so that the 8 k-values a lane needs for the permuted-t operand
