@@ -22,14 +22,6 @@ namespace ua {
 // where one of 8 waves waits as a whole.  h = 8, L = 4096, d = 128: forward 138 -> 115 us, key side 254 -> 230 and, with the stores of a
 // step left in flight over the next barrier, 186; column side 80 -> 70.
 constexpr int kAffWaves = 4;
-// Head and key group of a workgroup.  Every XCD gets whole heads (xcd_map).  A launch with one workgroup per key group runs the first
-// half of a head's groups from the longest sweep on and the second half from the shortest, so that the groups that share a
-// CU add up to the same length.
-__device__ __forceinline__ void aff_group(int n, int& bx, int& z) {
-  xcd_map(bx, z);
-  if ((int)gridDim.x == n && 2 * bx >= n) bx = n - 1 - (bx - n / 2);
-}
-
 // The pipeline macros of ua_fused.hpp are private to that header; these kernels use a two-stage loop of their own,
 // unrolled by two over two distinct LDS objects, and take one key group per workgroup or two of complementary length.
 // grid (Lp/NKEY or half of it, Z), NW waves; wave w owns keys 16*(NW*bx+w)..+15 and sweeps the 32-query blocks from its own on.
@@ -53,7 +45,7 @@ __global__ void __launch_bounds__(64 * kAffWaves) k_aff_fwd(const T* __restrict_
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
   const int n_kg = Lp / NKEY;
   int bx0, z;
-  aff_group(n_kg, bx0, z);
+  balanced_map(bx0, z);
   const GroupMasks gm = group_masks(lane);
   auto sweep = [&](const int bx) __attribute__((always_inline)) {
   const int nT = Lp / 32, sb16 = NW * bx + w, first = (NW / 2) * bx, own = sb16 >> 1;
@@ -302,7 +294,7 @@ __global__ void __launch_bounds__(64 * kAffWaves) k_aff_bwd_keys(const T* __rest
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
   const int n_kg = Lp / NKEY;
   int bx0, z;
-  aff_group(n_kg, bx0, z);
+  balanced_map(bx0, z);
   const int nTr = (L + 31) / 32;
   const GroupMasks gm = group_masks(lane);
   auto sweep = [&](const int bx) __attribute__((always_inline)) {
@@ -431,7 +423,7 @@ __global__ void __launch_bounds__(64 * kAffWaves) k_aff_bwd_cols(const T* __rest
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
   const int n_blk = Lp / (16 * NW);
   int bx0, z;
-  aff_group(n_blk, bx0, z);
+  balanced_map(bx0, z);
   auto sweep = [&](const int jt) __attribute__((always_inline)) {
     const int tq = NW * jt + w;
     if (16 * NW * jt >= L) return;                     // padding positions only

@@ -228,6 +228,27 @@ __device__ __forceinline__ void xcd_map(int& bx, int& by) {
     bx = slot % gx;
   }
 }
+// The same for kernels of which (at least) two workgroups fit a CU and whose sweeps shorten with bx, in launches of one to two
+// workgroups per CU: the first 256 take the longest sweeps, the others start with the shortest, so that the two that
+// share a CU add up to about the same length.  Plain order gives a CU two long ones: key side of the backward in 4-wave workgroups at
+// h = 16, L = 2048, d = 64 112 us, balanced 87.
+__device__ __forceinline__ void balanced_map(int& bx, int& by) {
+  constexpr int kCUs = 256;
+  const int gx = gridDim.x, gy = gridDim.y, total = gx * gy;
+  xcd_map(bx, by);
+  if (total <= kCUs || total > 2 * kCUs) return;
+  const int n = blockIdx.x + gx * blockIdx.y;
+  if ((gy & 7) == 0) {                         // every XCD its own heads
+    const int heads = gy >> 3, per_xcd = total >> 3, slot = n >> 3;
+    const int rank = slot < kCUs / 8 ? slot : per_xcd - 1 - (slot - kCUs / 8);
+    bx = rank / heads;
+    by = (n & 7) + 8 * (rank % heads);
+  } else {
+    const int rank = n < kCUs ? n : total - 1 - (n - kCUs);
+    bx = rank / gy;
+    by = rank % gy;
+  }
+}
 __device__ __forceinline__ long rows_out(const RowsOut& o, int z) {
   return (long)(z / (o.H * o.R)) * o.sb + (long)(z / o.R % o.H) * o.sh + (long)(z % o.R) * o.sr;
 }

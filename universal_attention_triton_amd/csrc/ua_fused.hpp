@@ -643,7 +643,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
 // (maximum, sum, O) of a slot are combined through LDS.  Key tiles are visited from the diagonal backwards.
 // Bound by the matrix pipe: three products of 16x16x4 instructions (32 cycles each).  A launch lasts as long as its longest workgroup, so
 // the workgroups are small (4 waves, 32 or 16 queries) and the waves of a block share its sweep: with 128 queries per workgroup and
-// no split b = 1, h = 8, L = 2048, d = 64 had 128 workgroups for 256 CUs, two waves of the longest one on each SIMD: 244 us, now 111;
+// no split b = 1, h = 8, L = 2048, d = 64 had 128 workgroups for 256 CUs, two waves of the longest one on each SIMD: 244 us, now 95;
 // h = 4, L = 512, d = 64 (four splits) 63 -> 16.
 // A split whose keys all lie after a query leaves the maximum -1e30 there, and its (finite) sums are weighted by 2^(-1e30 - max) = 0.
 // ---------------------------------------------------------------------------------------------
@@ -666,7 +666,7 @@ __global__ void __launch_bounds__(64 * NW) k_fwd_split(RowsOut orow_arg, const f
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
   const int slot = w / KS, ks = w % KS;
   int bx, zq;
-  xcd_map(bx, zq);
+  balanced_map(bx, zq);
   const int zk = zq / R, nT16 = Lp / 16, jt = (int)gridDim.x - 1 - bx;      // heaviest first
   const int tq = NS * jt + slot, tbq = tq >> 1;              // Lp is a multiple of 128: every wave has a query block
   char* sPw = sPbuf + w * ST::BYTES;
@@ -1140,7 +1140,7 @@ __device__ __forceinline__ Frag<T> ld8_tr(const T* tile, int n, int lane) {
 // Key-stationary backward (fused mode).  grid (n or ceil(n / 2), Zk) with n = Lp/128 key groups g (the second form: groups
 // g and n - 1 - g one after the other, see the body); 8 waves; wave w owns keys 128g+16w..+15 and
 // sweeps the 32-query blocks from the last one down to its own; one (query block, query group) per step.
-// NW = 4 (float32): workgroups of 64 keys, see bwd2_mr; h = 8, L = 2048, d = 64 in 291 instead of 465 us.
+// NW = 4: workgroups of 64 keys for float32 (h = 8, L = 2048, d = 64 in 290 instead of 465 us) and for small launches, see bwd2_mr.
 // MR = more than one query group per kv head (the decay state of a query block then lives across steps).
 // ---------------------------------------------------------------------------------------------
 // CH: chunked operator (a.c a multiple of 64): the upstream gradient, delta and the normaliser depend on the key's chunk
@@ -1151,7 +1151,7 @@ template <class T, int D, int NST, bool MR, bool CH, bool TO, int NW = 8>
 __global__ void __launch_bounds__(64 * NW) k_bwd_keys2(BwdArgs<T> a) {
   using TN = Tile<T, 32, D>;
   using TT = Tile<T, D, 32>;
-  static_assert(NW == 8 || (NW == 4 && !CH && !TO), "4 waves: merged operator without tile exchange");
+  static_assert(NW == 8 || (NW == 4 && !CH), "4 waves: merged operator");
   constexpr int NK = D / 32, ND = D / 16;
   // merged operator with tile exchange: the bias comes from the fp16 tiles of k_carry2<BO> (a.Bt), one 1 KB tile per wave
   // and step after the stats row (the chunked operator keeps the carries C, and Dsuf for the recomputing query side)
@@ -1162,7 +1162,7 @@ __global__ void __launch_bounds__(64 * NW) k_bwd_keys2(BwdArgs<T> a) {
   constexpr int TILES = TR ? (CH ? 4 : 3) * TN::BYTES : (CH ? 4 : 3) * (TN::BYTES + TT::BYTES);
   // offsets of the second chunk's upstream tile (CH), natural and transposed
   constexpr int DO2 = TR ? 3 * TN::BYTES : 3 * TN::BYTES + 3 * TT::BYTES, DO2T = 4 * TN::BYTES + 3 * TT::BYTES;
-  constexpr int SB = TILES + (CH ? 2048 : 1024) + (BI ? 8 * 1024 : 0);
+  constexpr int SB = TILES + (CH ? 2048 : 1024) + (BI ? NW * 1024 : 0);
   // tiles of a stage: Kt, Q, dO | (!TR) KT, QT, dOT | (CH) dO, dOT of the workgroup's second chunk
   // stats row of a stage: [lse2: 32f][delta: 32f][ldest: 32f][unused: 32f][forward carries of the 128 keys: 128f]
   // (CH) followed by [lse2: 32f][delta: 32f] of the second chunk
@@ -1180,7 +1180,8 @@ __global__ void __launch_bounds__(64 * NW) k_bwd_keys2(BwdArgs<T> a) {
   // workgroups that draw their key groups from a queue) the same step is scheduled with nearly twice the LDS waits and the
   // kernel is slower than with a workgroup per key group.
   int bx0, zo;
-  xcd_map(bx0, zo);
+  if constexpr (NW == 4) balanced_map(bx0, zo);
+  else xcd_map(bx0, zo);
   const int n_kg = a.Lp / (16 * NW);
   auto sweep = [&](const int bx) __attribute__((always_inline)) {
   const int zk = zo / a.key_parts;
@@ -1260,6 +1261,11 @@ __global__ void __launch_bounds__(64 * NW) k_bwd_keys2(BwdArgs<T> a) {
   const long st_head = grp_tiles(Lp >> 5) << 10;                   // bytes of gradient tiles per head
   const long st_lane = StageT<bf16>::addr(perm32(16 * (sb16 & 1) + col), 8 * g);
 
+  // 4 waves (launches bound by the latency of a step): the tiles' stores stay in flight over the next barrier
+  constexpr bool LATE = TO && NW == 4;
+  bool stored = false;
+#undef UA_WAIT
+#define UA_WAIT() if constexpr (LATE) wait_loads_before_stores<MR ? 2 : 4>(stored); else wait_async_loads(); stored = false
 #define UA_ISSUE(s, base)                                                                   \
   {                                                                                         \
     const int tb_ = top - (s) / R;                                                          \
@@ -1416,6 +1422,7 @@ __global__ void __launch_bounds__(64 * NW) k_bwd_keys2(BwdArgs<T> a) {
       const Frag<T> bp = as_operand16<T>(P[0], P[1]), bs = as_operand16<T>(dS[0], dS[1]);
       if constexpr (TO) {     // the two halves of the operand are the two query tiles of the block
         // query tiles 2 tb and 2 tb + 1: their rows start tb + 1 tiles apart
+        if constexpr (LATE) stores_after_loads();
         char* p = reinterpret_cast<char*>(a.dS_st) + (zq0 + r) * st_head + (grp_tile(2 * tb, sb16 >> 1) << 10) + st_lane;
         __builtin_nontemporal_store(reinterpret_cast<const u32x2*>(&bs)[0], reinterpret_cast<u32x2*>(p));
         __builtin_nontemporal_store(reinterpret_cast<const u32x2*>(&bs)[1], reinterpret_cast<u32x2*>(p + 1024));
@@ -1491,6 +1498,7 @@ __global__ void __launch_bounds__(64 * NW) k_bwd_keys2(BwdArgs<T> a) {
       }
       __builtin_amdgcn_s_setprio(0);
     }
+    if constexpr (LATE) stored = true;
   };
   {
     // the last NW / 2 query blocks of the sweep hold the diagonal blocks of the waves
@@ -1501,6 +1509,8 @@ __global__ void __launch_bounds__(64 * NW) k_bwd_keys2(BwdArgs<T> a) {
     UA_PIPE_RANGE(nfast, total, total, UA_ISSUE, UA_COMPUTE_SLOW);
   }
 #undef UA_ISSUE
+#undef UA_WAIT
+#define UA_WAIT() wait_async_loads()
 #undef UA_COMPUTE_FAST
 #undef UA_COMPUTE_SLOW
   // epilogue
@@ -1547,7 +1557,7 @@ __global__ void __launch_bounds__(64 * NW) k_bwd_keys2(BwdArgs<T> a) {
 // Query-stationary backward (fused mode): dQ and the column side of dK, no atomics.
 // grid (Lp/(16 NS), Zk); NW = NS KS waves: NS slots of 16 queries x KS key splits; 64 keys per step (KS = 2: wave ks of a slot takes
 // half ks of them, and the two waves' sums are added through LDS at the end: float32, bound by the matrix pipe, in 4-wave workgroups of
-// 32 queries at d = 64: h = 8, L = 2048 392 -> 172 us).
+// 32 queries at d = 64: h = 8, L = 2048 392 -> 144 us).
 //   dQ[t,:] += sum_s dS[s,t] k_s        dkcol[u,:] += sum_s dg[s,u] k_s
 // dS^T and dg^T pass through a wave-private LDS tile to become A operands.  With r query groups the sweep is
 // repeated per group; dg is linear in dBias, so the groups' contributions to dkcol add up (the cross-tile
@@ -1576,7 +1586,8 @@ __global__ void __launch_bounds__(64 * NW) k_bwd_queries2(BwdArgs<T> a, int d) {
   // of query heads, one (kv head, query group) per workgroup: more, smaller workgroups; the column-side key gradient
   // is then written per query head and added up by k_bwd_finish
   int bx, zy;
-  xcd_map(bx, zy);
+  if constexpr (KS == 2) balanced_map(bx, zy);
+  else xcd_map(bx, zy);
   const int Lp = a.Lp, L = a.L, nT16 = Lp / 16, R = a.R;
   const bool split_r = a.split_r != 0;
   const int zk = split_r ? zy / R : zy, r_begin = split_r ? zy % R : 0, r_end = split_r ? r_begin + 1 : R;
@@ -1878,8 +1889,8 @@ __global__ void __launch_bounds__(64 * NW) k_bwd_queries2(BwdArgs<T> a, int d) {
 // ---------------------------------------------------------------------------------------------
 // HV: 32-key halves per step.  With one half a stage is 25 KB and two workgroups share a CU (the kernel only moves
 // bytes: more of them in flight, and one workgroup's prologue and epilogue under the other's stream).
-template <class T, int D, int NST, int HV>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(HV == 1 ? 4 : 2, HV == 1 ? 4 : 2)))
+template <class T, int D, int NST, int HV, int NW = 8>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HV == 1 ? 4 : 2, HV == 1 ? 4 : 2)))
 k_bwd_queries3(BwdArgs<T> a, int d) {
   static_assert(sizeof(T) == 2, "tiles are exchanged in 16-bit operand precision");
   static_assert(HV == 1 || HV == 2, "one or two key halves per step");
@@ -1887,26 +1898,27 @@ k_bwd_queries3(BwdArgs<T> a, int d) {
   using ST = StageT<T>;
   constexpr int ND = D / 16;
   // stage: [KT half 0]([KT half 1])[per wave: dS half 0, (dS half 1,) dG half 0(, dG half 1)][reach of 4 key tiles]
-  constexpr int TILES = HV * TT::BYTES, WAVE = 2 * HV * ST::BYTES, SB = TILES + 8 * WAVE + 1024;
+  constexpr int TILES = HV * TT::BYTES, WAVE = 2 * HV * ST::BYTES, SB = TILES + NW * WAVE + 1024;
   UA_STAGES(SB);
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
   int bx0, zq;
-  xcd_map(bx0, zq);
+  if constexpr (NW == 4) balanced_map(bx0, zq);
+  else xcd_map(bx0, zq);
   const int Lp = a.Lp, L = a.L, nT16 = Lp / 16, R = a.R, zk = zq / R, r = zq % R;
   // chunked operator with live (query, later chunk) pairs: their tiles are not exchanged, k_bwd_queries2 runs instead
   if (a.chunked && !a.skip_masked && *a.masked_nz != 0) return;
-  const int n_blk = Lp / 128;
+  const int n_blk = Lp / (16 * NW);
   // two query blocks of complementary length per workgroup, the body expanded once per block (see k_bwd_keys2)
   auto sweep = [&](const int jt) __attribute__((always_inline)) {
-  const int tq = 8 * jt + w, tbq = tq >> 1;
-  Stager<TT, 8> stT;
+  const int tq = NW * jt + w, tbq = tq >> 1;
+  Stager<TT, NW> stT;
   stT.init(w, lane, Lp * (long)sizeof(T), D);
   f32x4 dQ[ND], dKc[ND];
 #pragma unroll
   for (int n = 0; n < ND; ++n) { dQ[n] = (f32x4){0, 0, 0, 0}; dKc[n] = (f32x4){0, 0, 0, 0}; }
   const T* KTz = a.KT + (long)zk * D * Lp;
-  const int n_kt = (4 * jt + 4) / HV;                  // steps of 32 HV keys
-  const int kt_min = (first_key_tile(a.reach + zk * nT16, 4 * jt, lane) >> (HV == 2 ? 2 : 1)) & ~1;
+  const int n_kt = (NW / 2) * (jt + 1) / HV;                  // steps of 32 HV keys
+  const int kt_min = (first_key_tile(a.reach + zk * nT16, (NW / 2) * jt, lane) >> (HV == 2 ? 2 : 1)) & ~1;
   // this lane's 16 bytes of the wave's tiles of key half h: base + h * 1024
   const long st_head = grp_tiles(Lp >> 5) << 10;
   const char* pS = reinterpret_cast<const char*>(a.dS_st) + (long)zq * st_head + (grp_tile(tq, 0) << 10) + 16 * lane;
@@ -1926,12 +1938,12 @@ k_bwd_queries3(BwdArgs<T> a, int d) {
     if (HV == 2) issue_row_nt(mine_ + ST::BYTES, pS + h_ + 8192);                                        \
     issue_row_nt(mine_ + HV * ST::BYTES, pG + h_);                                                               \
     if (HV == 2) issue_row_nt(mine_ + 3 * ST::BYTES, pG + h_ + 8192);                                    \
-    if (w == 0) issue_row((base) + TILES + 8 * WAVE, reach_z + 4 * (HV == 2 ? (s) : (s) >> 1));                  \
+    if (w == 0) issue_row((base) + TILES + NW * WAVE, reach_z + 4 * (HV == 2 ? (s) : (s) >> 1));                  \
   }
 #define UA_COMPUTE(s, base) bq_step((s), (base))
   auto bq_step = [&] __device__ (int kti, char* base) {
     char* mine = base + TILES + w * WAVE;
-    const int* rch = reinterpret_cast<const int*>(base + TILES + 8 * WAVE);
+    const int* rch = reinterpret_cast<const int*>(base + TILES + NW * WAVE);
 #pragma unroll
     for (int kq = 0; kq < HV; ++kq) {
       // the half's two 16-key tiles: visited by k_bwd_keys2 (hence written) iff not after the queries and in reach
@@ -1963,8 +1975,8 @@ k_bwd_queries3(BwdArgs<T> a, int d) {
   static_assert(NST == 2, "the epilogue stages its tiles in both stage buffers");
   __syncthreads();                      // every wave is done with the stages
   constexpr int RS = 64 + 4;            // floats per staged row: the four row groups of a store hit different banks
-  static_assert(4 * 16 * RS * 4 <= SB, "staging area");
-  float* xs = reinterpret_cast<float*>((w < 4 ? stage0 : stage1) + (w & 3) * (16 * RS * 4));
+  static_assert(NW / 2 * 16 * RS * 4 <= SB, "staging area");
+  float* xs = reinterpret_cast<float*>((w < NW / 2 ? stage0 : stage1) + (w % (NW / 2)) * (16 * RS * 4));
   const bool vec_ok = (d & 3) == 0 && ((reinterpret_cast<uintptr_t>(a.dq_out) | reinterpret_cast<uintptr_t>(a.dk_out)) & 7) == 0 &&
                       ((a.q_rows.sb | a.q_rows.sh | a.q_rows.sr | a.q_rows.st | a.kv_rows.sb | a.kv_rows.sh | a.kv_rows.st) & 3) == 0;
   T* const dq_z = a.dq_out + rows_out(a.q_rows, zq);

@@ -29,6 +29,11 @@ UA_INST(bf16, 64, 2) UA_INST(bf16, 128, 2) UA_INST(float, 64, 1) UA_INST(float, 
   template __global__ void k_bwd_keys2<float, D, 1, true, false, false, 4>(BwdArgs<float>);
 UA_INST4(64) UA_INST4(128)
 #undef UA_INST4
+#define UA_INST4(D) \
+  template __global__ void k_bwd_keys2<bf16, D, 2, false, false, true, 4>(BwdArgs<bf16>); \
+  template __global__ void k_bwd_keys2<bf16, D, 2, true, false, true, 4>(BwdArgs<bf16>);
+UA_INST4(64) UA_INST4(128)
+#undef UA_INST4
 template __global__ void k_bwd_keys2<bf16, 64, 2, false, false, true>(BwdArgs<bf16>);
 template __global__ void k_bwd_keys2<bf16, 64, 2, true, false, true>(BwdArgs<bf16>);
 template __global__ void k_bwd_keys2<bf16, 128, 2, false, false, true>(BwdArgs<bf16>);
@@ -51,8 +56,18 @@ static hipError_t bwd2_mr(const BwdArgs<T>& a, int Lp, int Zk, hipStream_t s, in
       return hipGetLastError();
     }
   }
-  // two key groups per workgroup once every CU gets at least two of the single ones
-  const int n_kg = Lp / 128, gx = paired_items(n_kg, (long)n_kg * Zk >= 2 * device_cus(), pair);
+  // bf16, up to one 8-wave workgroup per CU: the latency of a step bounds the launch, and twice as many 4-wave workgroups have shorter steps
+  // (1.8 us against 2.2) and fill each other's gaps: h = 8, L = 1024, d = 128 (64 of 8 waves) 70 -> 57 us, h = 16, L = 2048 (256) 138 ->
+  // 121.  With more, pairs of 8-wave workgroups are as fast (384: 273 and 275 us) and sweep the tiles half as often.
+  if constexpr (TO && !CH && D <= 128) {
+    if ((long)(Lp / 128) * Zk <= device_cus()) {
+      hipLaunchKernelGGL((k_bwd_keys2<T, D, NST, MR, CH, TO, 4>), dim3(Lp / 64, Zk), dim3(256), 0, s, a);
+      return hipGetLastError();
+    }
+  }
+  // two key groups per workgroup once there are more of the single ones than CUs: the launch is one round of equal workgroups
+  // instead of a second one behind the longest (h = 12, L = 4096, d = 128, 384 key groups: 476 -> 273 us)
+  const int n_kg = Lp / 128, gx = paired_items(n_kg, (long)n_kg * Zk > device_cus(), pair);
   hipLaunchKernelGGL((k_bwd_keys2<T, D, NST, MR, CH, TO>), dim3(gx, Zk), dim3(512), 0, s, a);
   return hipGetLastError();
 }
@@ -124,6 +139,8 @@ hipError_t launch_bwd_queries(int dtype, int D, const BwdArgsV& a, int d, int Zk
   return D == 64 ? bwdq_t<float, 64, 1>(a, d, Zk, s) : bwdq_t<float, 128, 1>(a, d, Zk, s);
 }
 
+template __global__ void k_bwd_queries3<bf16, 64, 2, 1, 4>(BwdArgs<bf16>, int);
+template __global__ void k_bwd_queries3<bf16, 128, 2, 1, 4>(BwdArgs<bf16>, int);
 template __global__ void k_bwd_queries3<bf16, 64, 2, 1>(BwdArgs<bf16>, int);
 template __global__ void k_bwd_queries3<bf16, 128, 2, 1>(BwdArgs<bf16>, int);
 template __global__ void k_bwd_queries3<bf16, 64, 2, 2>(BwdArgs<bf16>, int);
@@ -135,6 +152,12 @@ hipError_t launch_bwd_queries_from_tiles(int D, const BwdArgsV& v, int d, int Zq
   // single ones, two once it gets four; steps of 64 keys: one block per workgroup
   const int n_blk = v.Lp / 128;
   const long n_wg = (long)n_blk * Zq;
+  // under two per CU: twice as many workgroups of 4 waves (h = 8, L = 1024, d = 128: 34.7 -> 30.8 us; h = 12, L = 4096, d = 64: 134 -> 122)
+  if (D <= 128 && n_wg < 2L * device_cus() && variant != 1) {
+    if (D == 64) hipLaunchKernelGGL((k_bwd_queries3<bf16, 64, 2, 1, 4>), dim3(v.Lp / 64, Zq), dim3(256), 0, s, a, d);
+    else hipLaunchKernelGGL((k_bwd_queries3<bf16, 128, 2, 1, 4>), dim3(v.Lp / 64, Zq), dim3(256), 0, s, a, d);
+    return hipGetLastError();
+  }
   const bool half_steps = !(variant == 1 && D != 256);
   const int gx = !half_steps ? n_blk
                  : (n_blk % 4 == 0 && n_wg >= 8L * device_cus()) ? n_blk / 4
