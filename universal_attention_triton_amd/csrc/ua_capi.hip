@@ -120,9 +120,12 @@ int heuristic_variant(const ua_desc& d, int slot) {
   const long Zk = (long)d.b * d.h, Zq = Zk * d.r;
   const int Lp = (int)align_up((size_t)d.L, 128);
   switch (slot) {
-    case UA_TUNE_CARRY: {    // 4-wave workgroups won at every tuned shape; two key groups each when the single ones make
-      const long n4 = Zk * (Lp / 64);      // one to four rounds of the 1024 resident workgroups
-      return (n4 >= 1024 && n4 < 4096) ? 2 : 1;
+    case UA_TUNE_CARRY: {
+      // 4-wave workgroups won at every tuned shape.  Up to eight per CU all of them run at once, in balanced order (k_carry2); above, the
+      // order cannot balance them and two key groups of complementary length each win until there are many rounds (L = 4096, d = 128,
+      // 2048 of them 182 us against 195 as pairs, 2304 302 against 286).
+      const long n4 = Zk * (Lp / 64);
+      return (n4 > 2048 && n4 < 4096) ? 2 : 1;
     }
     case UA_TUNE_FWD_TILES: {
       // 4-wave workgroups (128 / RB queries, two per CU) win once there are three per CU: b = 1 h = 8 r = 4 L = 4096 d = 128 (1024 of

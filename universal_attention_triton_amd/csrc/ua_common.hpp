@@ -232,19 +232,26 @@ __device__ __forceinline__ void xcd_map(int& bx, int& by) {
 // workgroups per CU: the first 256 take the longest sweeps, the others start with the shortest, so that the two that
 // share a CU add up to about the same length.  Plain order gives a CU two long ones: key side of the backward in 4-wave workgroups at
 // h = 16, L = 2048, d = 64 112 us, balanced 87.
+// ROUNDS: workgroups of the kernel that fit a CU; launches of more than two per CU go round by round, every second round in reverse.
+template <int ROUNDS = 2>
 __device__ __forceinline__ void balanced_map(int& bx, int& by) {
   constexpr int kCUs = 256;
   const int gx = gridDim.x, gy = gridDim.y, total = gx * gy;
   xcd_map(bx, by);
-  if (total <= kCUs || total > 2 * kCUs) return;
+  if (total <= kCUs || total > ROUNDS * kCUs) return;
   const int n = blockIdx.x + gx * blockIdx.y;
+  // place in the order of falling length of item i of `all`, `cus` of them running at a time
+  auto rank_of = [&] __device__ (int i, int all, int cus) {
+    if (ROUNDS == 2 || all <= 2 * cus) return i < cus ? i : all - 1 - (i - cus);
+    const int r0 = i / cus * cus;
+    return (i / cus) & 1 ? r0 + min(cus, all - r0) - 1 - (i - r0) : i;
+  };
   if ((gy & 7) == 0) {                         // every XCD its own heads
-    const int heads = gy >> 3, per_xcd = total >> 3, slot = n >> 3;
-    const int rank = slot < kCUs / 8 ? slot : per_xcd - 1 - (slot - kCUs / 8);
+    const int heads = gy >> 3, rank = rank_of(n >> 3, total >> 3, kCUs / 8);
     bx = rank / heads;
     by = (n & 7) + 8 * (rank % heads);
   } else {
-    const int rank = n < kCUs ? n : total - 1 - (n - kCUs);
+    const int rank = rank_of(n, total, kCUs);
     bx = rank / gy;
     by = rank % gy;
   }

@@ -111,13 +111,14 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
   constexpr int NK = D / 32, SB = TN::BYTES + 1024;   // tile + [ldest of the block: 32 floats]
   UA_STAGES(SB);
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
-  // A launch of half as many workgroups has each sweep two key groups, bx and (number of key groups - 1 - bx), one after
-  // the other with the body expanded once per key group (see k_bwd_keys2).  It pays in small launches (b = 2, h = 16,
-  // L = 2048, d = 64: 0.074 -> 0.056 ms) and costs in large ones (b = 1, h = 32, L = 8192: 0.70 -> 0.83 ms), so it is a
-  // variant of the tuning slot.
+  // One key group per workgroup: up to eight of the 4-wave workgroups run on a CU at once, ordered so that their sweeps add up to the same
+  // length on every CU (b = 2, h = 16, L = 2048, d = 64: 43 us).  A launch of half as many workgroups has each sweep two key groups, bx and
+  // (number of key groups - 1 - bx), one after the other with the body expanded once per key group (see k_bwd_keys2): equal
+  // workgroups in any order (52 us there), for launches of a few uneven rounds (h = 36, L = 4096, d = 128: 302 -> 286 us).
   int bx0, z;
-  xcd_map(bx0, z);
   const int n_kg = Lp / (16 * NW);
+  if (NW == 4 && (int)gridDim.x == n_kg) balanced_map<8>(bx0, z);
+  else xcd_map(bx0, z);
   __shared__ int n_dead;
   __shared__ float red[2][NW];
   auto sweep = [&](const int bx) __attribute__((always_inline)) {

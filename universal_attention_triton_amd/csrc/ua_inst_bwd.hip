@@ -29,6 +29,8 @@ UA_INST(bf16, 64, 2) UA_INST(bf16, 128, 2) UA_INST(float, 64, 1) UA_INST(float, 
   template __global__ void k_bwd_keys2<float, D, 1, true, false, false, 4>(BwdArgs<float>);
 UA_INST4(64) UA_INST4(128)
 #undef UA_INST4
+template __global__ void k_bwd_keys2<float, 64, 2, false, false, false, 4>(BwdArgs<float>);
+template __global__ void k_bwd_keys2<float, 64, 2, true, false, false, 4>(BwdArgs<float>);
 #define UA_INST4(D) \
   template __global__ void k_bwd_keys2<bf16, D, 2, false, false, true, 4>(BwdArgs<bf16>); \
   template __global__ void k_bwd_keys2<bf16, D, 2, true, false, true, 4>(BwdArgs<bf16>);
@@ -51,6 +53,12 @@ static hipError_t bwd2_mr(const BwdArgs<T>& a, int Lp, int Zk, hipStream_t s, in
   // LDS of a CU, which pays while the workgroups of 8 waves are fewer than two per CU and their longest bounds the launch (h = 8,
   // L = 3000: step 3.27 -> 1.92 ms) and costs beyond (h = 16, L = 8192: 18.6 -> 20.8).
   if constexpr (sizeof(T) == 4 && !CH) {
+    if constexpr (D == 64) {
+      if ((long)(Lp / 64) * Zk <= device_cus()) {       // one per CU: two stages (h = 8, L = 2048: step 605 -> 596 us)
+        hipLaunchKernelGGL((k_bwd_keys2<T, D, 2, MR, CH, TO, 4>), dim3(Lp / 64, Zk), dim3(256), 0, s, a);
+        return hipGetLastError();
+      }
+    }
     if (D == 64 || (long)(Lp / 128) * Zk < 2L * device_cus()) {
       hipLaunchKernelGGL((k_bwd_keys2<T, D, NST, MR, CH, TO, 4>), dim3(Lp / 64, Zk), dim3(256), 0, s, a);
       return hipGetLastError();
