@@ -256,6 +256,19 @@ __device__ __forceinline__ void balanced_map(int& bx, int& by) {
     by = rank % gy;
   }
 }
+// Longest sweeps of all heads first (bx = 0 is the longest): for launches of between one and two workgroups per CU that run one per CU,
+// where a CU takes its second one as soon as its first ends.
+__device__ __forceinline__ void longest_first_map(int& bx, int& by) {
+  const int gx = gridDim.x, gy = gridDim.y, n = blockIdx.x + gx * blockIdx.y;
+  if ((gy & 7) == 0) {                         // every XCD its own heads (see xcd_map)
+    const int heads = gy >> 3, slot = n >> 3;
+    bx = slot / heads;
+    by = (n & 7) + 8 * (slot % heads);
+  } else {
+    bx = n / gy;
+    by = n % gy;
+  }
+}
 __device__ __forceinline__ long rows_out(const RowsOut& o, int z) {
   return (long)(z / (o.H * o.R)) * o.sb + (long)(z / o.R % o.H) * o.sh + (long)(z % o.R) * o.sr;
 }

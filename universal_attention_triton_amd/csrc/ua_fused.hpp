@@ -1181,9 +1181,10 @@ __global__ void __launch_bounds__(64 * NW) k_bwd_keys2(BwdArgs<T> a) {
   // workgroups that draw their key groups from a queue) the same step is scheduled with nearly twice the LDS waits and the
   // kernel is slower than with a workgroup per key group.
   int bx0, zo;
-  if constexpr (NW == 4) balanced_map(bx0, zo);
-  else xcd_map(bx0, zo);
   const int n_kg = a.Lp / (16 * NW);
+  if constexpr (NW == 4) balanced_map(bx0, zo);
+  else if ((int)gridDim.x == n_kg) longest_first_map(bx0, zo);
+  else xcd_map(bx0, zo);
   auto sweep = [&](const int bx) __attribute__((always_inline)) {
   const int zk = zo / a.key_parts;
   const int Lp = a.Lp, L = a.L, nT16 = Lp / 16, R = MR ? a.R / a.key_parts : 1;

@@ -73,9 +73,9 @@ static hipError_t bwd2_mr(const BwdArgs<T>& a, int Lp, int Zk, hipStream_t s, in
       return hipGetLastError();
     }
   }
-  // two key groups per workgroup once there are more of the single ones than CUs: the launch is one round of equal workgroups
-  // instead of a second one behind the longest (h = 12, L = 4096, d = 128, 384 key groups: 476 -> 273 us)
-  const int n_kg = Lp / 128, gx = paired_items(n_kg, (long)n_kg * Zk > device_cus(), pair);
+  // two key groups per workgroup once every CU gets at least two of the single ones; with fewer the kernel takes the longest ones of all
+  // heads first
+  const int n_kg = Lp / 128, gx = paired_items(n_kg, (long)n_kg * Zk >= 2 * device_cus(), pair);
   hipLaunchKernelGGL((k_bwd_keys2<T, D, NST, MR, CH, TO>), dim3(gx, Zk), dim3(512), 0, s, a);
   return hipGetLastError();
 }
