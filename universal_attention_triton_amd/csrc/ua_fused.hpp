@@ -1904,7 +1904,7 @@ k_bwd_queries3(BwdArgs<T> a, int d) {
   UA_STAGES(SB);
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
   int bx0, zq;
-  if constexpr (NW == 4) balanced_map(bx0, zq);
+  if constexpr (NW == 4) balanced_map<4>(bx0, zq);
   else xcd_map(bx0, zq);
   const int Lp = a.Lp, L = a.L, nT16 = Lp / 16, R = a.R, zk = zq / R, r = zq % R;
   // chunked operator with live (query, later chunk) pairs: their tiles are not exchanged, k_bwd_queries2 runs instead

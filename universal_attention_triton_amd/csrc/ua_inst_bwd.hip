@@ -160,7 +160,7 @@ hipError_t launch_bwd_queries_from_tiles(int D, const BwdArgsV& v, int d, int Zq
   // single ones, two once it gets four; steps of 64 keys: one block per workgroup
   const int n_blk = v.Lp / 128;
   const long n_wg = (long)n_blk * Zq;
-  // under two per CU: twice as many workgroups of 4 waves (h = 8, L = 1024, d = 128: 34.7 -> 30.8 us; h = 12, L = 4096, d = 64: 134 -> 122)
+  // under two per CU: twice as many workgroups of 4 waves (h = 8, L = 1024, d = 128: 34.7 -> 30.8 us; h = 12, L = 4096, d = 64: 134 -> 114)
   if (D <= 128 && n_wg < 2L * device_cus() && variant != 1) {
     if (D == 64) hipLaunchKernelGGL((k_bwd_queries3<bf16, 64, 2, 1, 4>), dim3(v.Lp / 64, Zq), dim3(256), 0, s, a, d);
     else hipLaunchKernelGGL((k_bwd_queries3<bf16, 128, 2, 1, 4>), dim3(v.Lp / 64, Zq), dim3(256), 0, s, a, d);
